@@ -56,14 +56,14 @@ enum { SR_PREC_F64 = 0, SR_PREC_SPLIT = 1 };
 
 /*
  * Sweep of the split path.  SR_SWEEP_DIRECT forms every phase in FP64.
- * SR_SWEEP_RECURRENCE, for grids that declare a constant omega_step, forms
- * exp(i omega tau) in FP64/FP32 for one omega per thread and advances it to the
- * thread's other omegas by complex multiplication, and sweeps only the steps
- * that keep some omega of each 64-omega run.  Both apply the |dphase| < pi
- * filter as the equivalent threshold |omega| < pi/|tau_s - tau_{s-1}|.
- * SR_SWEEP_AUTO selects the recurrence on linear grids and the direct sweep
- * otherwise.  The FP64 path always sweeps directly and filters
- * exactly as the reference does.
+ * SR_SWEEP_RECURRENCE, for grids that declare a constant omega_step, forms the
+ * phases of groups of 32 omegas from a few phases per step by the addition
+ * theorems and sums the steps as matrix products (two fp16 words per FP32
+ * factor, FP32 accumulation, FP64 sums).  Both apply the |dphase| < pi filter as
+ * the equivalent threshold |omega| < pi/|tau_s - tau_{s-1}|.
+ * SR_SWEEP_AUTO selects it on linear grids (far field: of more than 64 omegas)
+ * and the direct sweep otherwise.  The FP64 path always sweeps directly and
+ * filters exactly as the reference does.
  */
 enum { SR_SWEEP_AUTO = 0, SR_SWEEP_DIRECT = 1, SR_SWEEP_RECURRENCE = 2 };
 
@@ -128,7 +128,8 @@ typedef struct sr_opts {
   int32_t precision;        /* SR_PREC_* */
   int32_t omega_per_lane;   /* 0 = tuned, else 1, 2 or 4; a value the variant lacks
                                falls back: split direct 1, 2, 4 far / 1, 2 near, else 1;
-                               recurrence 2, 4 far / 2 near, else 2; f64 1, 2, else 1 */
+                               recurrence 2, 4 far (tiles of up to 256, 512 omegas)
+                               / 2 near (128), else 2; f64 1, 2, else 1 */
   int32_t waves_per_block;  /* 0 = tuned, else 1, 2 or 4 */
   int32_t slices;           /* 0 = tuned, else 1..32 particle slices */
   int32_t persistent;       /* 0 = one block per tile; >0 = that many blocks loop over tiles */

@@ -40,14 +40,8 @@
 //                     revolutions -> v_fract_f64 -> v_sin_f32/v_cos_f32, the
 //                     filter in its threshold form |omega|/2pi < 1/(2|dtau|),
 //                     FP32 sums with a Kahan fold per swept segment.
-//       split rec     (linear grids) the thread's M omegas differ by T*domega,
-//                     so exp(i omega_k tau) is advanced from k to k+1 by one
-//                     complex multiply with exp(i T domega tau) (computed per
-//                     step in the stage).  The tile's steps are put in an order
-//                     in which every 64-omega run finds the steps keeping any of
-//                     its omegas first (a stable counting sort), so each wave
-//                     sweeps only those, stops the rotation chain at its last
-//                     kept run and masks only that run.
+//     Split spectra on linear grids run another kernel, factored.h: there the
+//     sums over the steps are matrix products of a few sines per step.
 //   * Records: with one snapshot and one output each thread sums its points
 //     over the block's particles in LDS and writes once; otherwise outputs are
 //     read-modify-written per particle record by the one thread that owns
@@ -72,6 +66,8 @@
 
 #include "synchrad_amd.h"
 #include "common.h"
+#include "tile_params.h"
+#include "factored.h"
 
 namespace sr {
 
@@ -97,54 +93,6 @@ enum { SWEEP_DIRECT = 0, SWEEP_REC = 1 };
 
 template <int V>
 using IC = std::integral_constant<int, V>;
-
-struct KParams {
-  // tracks (CSR); offsets == nullptr selects the single-particle form
-  const int64_t *offsets;
-  const double *x, *y, *z, *ux, *uy, *uz;
-  const double *weight;
-  const uint32_t *it_start, *it_end, *it_snaps;
-  uint32_t n_snaps, snaps_stride;
-  double dt;
-  int64_t single_n;
-  double single_w;
-  uint32_t single_its, single_ite;
-  // grid
-  int32_t comp;
-  uint32_t n_omega, n_theta, n_phi;
-  const double *omega, *sin_t, *cos_t, *radius, *sin_p, *cos_p;
-  const double *screen_y;   // near, Cartesian screen: P = (radius[i], screen_y[j], L)
-  double l_screen;
-  double omega_step;        // rec sweep: omega[i+1] - omega[i]
-  const double *form_factor;
-  int64_t n_grid;
-  // outputs (slices > 1: scratch[q][c] replaces out[c])
-  int32_t n_out;
-  double *out[kMaxOut];
-  double *scratch;
-  // 1: one snapshot and one output -- each thread sums its points over the
-  // block's particles in LDS and adds the sum to the output once
-  int32_t acc_lds;
-  // per-particle outputs (the adjoint's fields): particle ip writes at
-  // (ip - part_base) * part_stride past the usual index; 0 otherwise
-  int64_t part_base, part_stride;
-  // direction-independent step data from k_step_prep, or nullptr (the stage
-  // then computes it), one record per sample: far [n_points][a_x, a_y, a_z,
-  // bbar_x, bbar_y, bbar_z] (48 B, 16-byte aligned), near [n_points][b_x, b_y,
-  // b_z].  One base address and fixed offsets: the stage reads a record with
-  // three 16-byte loads and keeps no per-array base registers
-  const double *pre;
-  int64_t n_points;
-  // tiling
-  uint32_t n_chunks;
-  uint32_t n_dir;
-  UDiv div_chunks, div_dir, div_theta;   // by n_chunks, n_dir, n_theta (tiles < 2^31)
-  int32_t slices;
-  int64_t n_tiles;
-  int64_t slice_lo[kMaxSlices + 1];
-  // launch order of the tiles (heaviest first), or nullptr: index order
-  const int32_t *tile_order;
-};
 
 // ---------------------------------------------------------------------------
 // the tile kernel
@@ -222,27 +170,14 @@ constexpr int amp_words() {
 }
 
 // Dynamic LDS before the Kahan state: one tile of T staged steps -- tau
-// (double), the split threshold (double), the recurrence rotation (2 floats)
-// and the amplitude words -- sized by the launched block, so that one-wave
-// blocks do not hold a 256-step tile's LDS.
-template <int MODE, int PREC, int SWEEP>
+// (double), the split threshold (double) and the amplitude words -- sized by the
+// launched block, so that one-wave blocks do not hold a 256-step tile's LDS.
+template <int MODE, int PREC>
 constexpr size_t stage_lds_bytes(int T) {
   constexpr bool split = PREC == SR_PREC_SPLIT;
-  return (size_t)T * (sizeof(double) + (split ? sizeof(double) : 0) + (SWEEP == SWEEP_REC ? 2 * sizeof(float) : 0) +
+  return (size_t)T * (sizeof(double) + (split ? sizeof(double) : 0) +
                       amp_words<MODE, PREC>() * (split ? sizeof(float) : sizeof(double)));
 }
-
-// one staged step of the recurrence sweep (split): tau, threshold, the
-// rotation e^{i T domega tau} and the amplitude words in one 16-byte aligned
-// record (32 B far, 48 B near), so that the sweep reads a group of steps from
-// one base address with immediate offsets (the same bytes as the separate
-// arrays of the other sweeps)
-template <int NA>
-struct alignas(16) RecStep {
-  double tau, thr;
-  float er, ei;
-  float amp[NA];
-};
 
 // rows of a [n][T] LDS array: rows[c][j]
 template <typename X>
@@ -253,33 +188,13 @@ struct LdsRows {
 };
 
 // Register budget per variant, as the minimum number of waves each SIMD must
-// be able to hold: the split sweeps keep their Kahan state in LDS, so their
+// be able to hold: the split sweep keeps its Kahan state in LDS, so its
 // registers hold the partial sums of M omegas plus one staged step group.
-// (far recurrence with M = 2: 4 waves, measured 3% faster than 3 despite a
-// few spilled stage registers; the other recurrence variants spill heavily
-// at 4 and run at 2)
-#ifndef SR_REC_WAVES
-#define SR_REC_WAVES 3
-#endif
-#ifndef SR_REC_WAVES_FAR2
-#define SR_REC_WAVES_FAR2 4
-#endif
-#ifndef SR_REC_WAVES_FAR4
-#define SR_REC_WAVES_FAR4 2
-#endif
-// recurrence groups of 4 steps: all base sin/cos first, then the sums
-#ifndef SR_REC_PIPE
-#define SR_REC_PIPE 1
-#endif
 #ifndef SR_WAVE_ROTATE
 #define SR_WAVE_ROTATE 1
 #endif
 #ifndef SR_DIRECT_WAVES
 #define SR_DIRECT_WAVES 3
-#endif
-// split stage: hardware FP64 reciprocal instead of IEEE division
-#ifndef SR_SPLIT_RCP
-#define SR_SPLIT_RCP 1
 #endif
 // split direct sweep in 4-step groups
 #ifndef SR_DIRECT_GROUP
@@ -298,56 +213,23 @@ struct LdsRows {
 #ifndef SR_F64_NEAR_WAVES2
 #define SR_F64_NEAR_WAVES2 SR_F64_WAVES2
 #endif
-// Recurrence sweep: the steps of a tile are put in an order in which every
-// 64-omega run of the block finds the steps that keep any of its omegas first,
-// so a wave sweeps only those (a stable counting sort per tile).  The direct
-// sweep measured slower with it (the sort's registers cost it a wave per SIMD
-// and skipped steps are already cheap there), so it keeps the tile order.
-// recurrence sweep: a thread's third and fourth omegas by the three-term
-// recurrence of equally spaced angles instead of a complex multiplication
-#ifndef SR_REC_CHEB
-#define SR_REC_CHEB 1
-#endif
-#ifndef SR_COMPACT
-#define SR_COMPACT 1
-#endif
-// recurrence sweep: a step's previous retarded time tau_{s-1} comes from the
-// neighbouring thread's stage through LDS (1) instead of being recomputed
-// from the previous sample (0); the tile's first thread recomputes it.  Same
-// results; three global loads fewer per step (the HBM traffic is unchanged:
-// the neighbouring lane's load had brought those lines in)
-#ifndef SR_TAU_EXCHANGE
-#define SR_TAU_EXCHANGE 1
-#endif
-// 1: a step's bucket (the number of runs it keeps) by binary search over the
-// runs' sorted smallest |omega| (log2 R compares; +0.8 % on the betatron
-// launch, same buckets); 0: by comparing with every run
-#ifndef SR_BUCKET_SEARCH
-#define SR_BUCKET_SEARCH 1
-#endif
-
-template <int MODE, int PREC, int SWEEP, int M>
+template <int MODE, int PREC, int M>
 struct WavesPerEU {
   static constexpr int value =
       (PREC == SR_PREC_F64) ? (M == 2 ? (MODE == SR_MODE_NEAR ? SR_F64_NEAR_WAVES2 : SR_F64_WAVES2)
                                       : SR_F64_WAVES)
-      : (SWEEP == SWEEP_REC) ? ((MODE == SR_MODE_FAR && M == 2)   ? SR_REC_WAVES_FAR2
-                                : (MODE == SR_MODE_FAR && M == 4) ? SR_REC_WAVES_FAR4
-                                                                  : SR_REC_WAVES)
-                             : (M >= 4 ? 2 : SR_DIRECT_WAVES);
+                            : (M >= 4 ? 2 : SR_DIRECT_WAVES);
 };
 
 // PRE: the step data come from the pre-pass records (batch calls); without
 // them (the per-particle and no-allocation calls) the stage forms them from u
-template <int MODE, int PREC, int SWEEP, int M, bool PRE>
+template <int MODE, int PREC, int M, bool PRE>
 __global__ void __launch_bounds__(kMaxT)
-__attribute__((amdgpu_waves_per_eu(WavesPerEU<MODE, PREC, SWEEP, M>::value)))
+__attribute__((amdgpu_waves_per_eu(WavesPerEU<MODE, PREC, M>::value)))
 k_spectrum(const KParams p) {
-  static_assert(!(PREC == SR_PREC_F64 && SWEEP == SWEEP_REC), "recurrence sweep is split-only");
   static_assert(PREC == SR_PREC_SPLIT || M <= 2, "the FP64 sweep holds one or two omegas per thread");
   using Amp = typename std::conditional<PREC == SR_PREC_SPLIT, float, double>::type;
   constexpr bool kSplit = (PREC == SR_PREC_SPLIT);
-  constexpr bool kRec = (SWEEP == SWEEP_REC);
   // amplitude words per step.  Far: A is perpendicular to n
   // (n.A = c1 (1 - n.bbar) - c2 n.a = 0 with c1 = (n.a) c2^2), so it is kept
   // as its two components on e_theta, e_phi (the reference sums A_x, A_y, A_z;
@@ -355,22 +237,9 @@ k_spectrum(const KParams p) {
   constexpr int NA = amp_words<MODE, PREC>();
   constexpr int NC = (MODE == SR_MODE_FAR) ? 2 * NA : 6;   // real accumulators per omega
   constexpr int NP = (MODE == SR_MODE_FAR) ? NC : 12;      // split register partials per omega
-  constexpr bool kCompact = kSplit && kRec && (SR_COMPACT != 0);
-  // (the direct sweep has no step sort whose barriers it could share: it
-  // recomputes tau_{s-1}, which measured 0.5 % faster there)
-  constexpr bool kExch = kSplit && kRec && (SR_TAU_EXCHANGE != 0);
   constexpr int kMaxW = kMaxT / kWave;                 // waves per block
-  constexpr int kMaxRuns = kMaxW * 4;                  // 64-omega runs per block (M <= 4)
 
   extern __shared__ __align__(16) char s_dyn_raw[];
-  // compaction: smallest |omega|/2pi of each run, its rank, the per-wave
-  // bucket histogram, its scan, and the step count of each rank
-  __shared__ double s_wmin[kCompact ? kMaxRuns : 1];
-  __shared__ int s_rank[kCompact ? kMaxRuns : 1];
-  __shared__ double s_wsort[kCompact ? kMaxRuns : 1];   // s_wmin in rank order (ascending)
-  __shared__ int s_hist[kCompact ? kMaxRuns * kMaxW : 1];
-  __shared__ int s_off[kCompact ? kMaxRuns * kMaxW : 1];
-  __shared__ int s_cntb[kCompact ? kMaxRuns + 1 : 1];
   // FP64 sin/cos table (sincos_table) and the largest |omega| of the grid
   constexpr bool kTab = !kSplit && (SR_F64_TABLE != 0);
   __shared__ double2 s_sct[kTab ? kSinCosTab : 1];
@@ -398,15 +267,12 @@ k_spectrum(const KParams p) {
     __syncthreads();
     for (int w = 0; w < W; w++) om_abs_max = fmax(om_abs_max, s_wmax[w]);
   }
-  // dynamic LDS: the staged tile (recurrence: s_rec[T]; else s_tau[T],
-  // s_thr[T] (split), s_amp[NA][T]), then the Kahan state, then the particle sums
-  static_assert(!kRec || sizeof(RecStep<NA>) == 2 * sizeof(double) + (2 + NA) * sizeof(float),
-                "a recurrence record holds exactly the staged step's bytes");
-  RecStep<NA> *const s_rec = (RecStep<NA> *)s_dyn_raw;
+  // dynamic LDS: the staged tile (s_tau[T], s_thr[T] (split), s_amp[NA][T]), then
+  // the Kahan state, then the particle sums
   double *const s_tau = (double *)s_dyn_raw;
   double *const s_thr = s_tau + T;
   const LdsRows<Amp> s_amp{(Amp *)(s_tau + (kSplit ? 2 : 1) * T), T};
-  float *const s_dyn = (float *)(s_dyn_raw + stage_lds_bytes<MODE, PREC, SWEEP>(T));
+  float *const s_dyn = (float *)(s_dyn_raw + stage_lds_bytes<MODE, PREC>(T));
   float *const s_ks = s_dyn + tid;                       // S[c*M+k] at s_ks[(c*M+k)*T]
   float *const s_kc = s_dyn + (size_t)NC * M * T + tid;  // C likewise
   // particle sums of the single output, k-th omega at s_acc[k*T]
@@ -414,7 +280,6 @@ k_spectrum(const KParams p) {
   const double dt = p.dt;
   const double dtInv = 1.0 / dt;
   const bool spheric = (p.comp == SR_COMP_SPHERIC || p.comp == SR_COMP_SPHERIC_COMPLEX);
-  const double rot_rev = (double)T * p.omega_step * kInv2Pi;   // revolutions of the k -> k+1 step
 
   for (int64_t ti = blockIdx.x; ti < p.n_tiles; ti += gridDim.x) {
     const uint32_t tile = p.tile_order ? (uint32_t)p.tile_order[ti] : (uint32_t)ti;
@@ -485,45 +350,7 @@ k_spectrum(const KParams p) {
       om_rev[k] = om[k] * kInv2Pi;
       omf[k] = (float)om[k];
     }
-    // rec sweep: the thread's base frequency in revolutions, the block's omega range
-    const double om0_rev = om_rev[0];
-    // range of |omega|/2pi over the block (linear grids: the run's end points)
-    double w_lo = 0.0, w_hi = 0.0;
-    bool rec_sortable = false;
     bool tile_wide = false;   // FP64: the tile's phases may reach kTabMaxPhase / 2
-    if (kRec) {
-      const int64_t first = (int64_t)chunk * T * M;
-      const int64_t last = min((int64_t)(chunk + 1) * T * M, (int64_t)p.n_omega) - 1;
-      const double a = p.omega[first] * kInv2Pi, b = p.omega[last] * kInv2Pi;
-      w_lo = (a * b <= 0.0) ? 0.0 : fmin(fabs(a), fabs(b));
-      w_hi = fmax(fabs(a), fabs(b));
-      rec_sortable = p.omega_step > 0.0 && a >= 0.0;
-    }
-    // compaction: run r = k*W + wave holds the k-th omegas of the wave's lanes;
-    // a step keeps some omega of run r iff s_wmin[r] < thr_s.  The recurrence
-    // sweep needs the thread's runs in ascending |omega| (a non-negative,
-    // increasing grid): then the runs a step keeps are a prefix k < K.
-    if (kCompact) {
-      __syncthreads();  // an earlier tile of this block is done with s_wmin, s_rank
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        double v = valid[k] ? fabs(om_rev[k]) : INFINITY;
-        for (int o = kWave / 2; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
-        if (lane == 0) s_wmin[k * W + vw] = v;
-      }
-      __syncthreads();
-      if (tid < W * M) {
-        const double mine = s_wmin[tid];
-        int rk = 0;
-        for (int r = 0; r < W * M; r++) {
-          const double o = s_wmin[r];
-          rk += (o < mine || (o == mine && r < tid)) ? 1 : 0;
-        }
-        s_rank[tid] = rk;
-        s_wsort[rk] = mine;
-      }
-      // published by the barrier that opens the first step tile
-    }
     // output c of this tile (slices: the slice's partial spectra), formed where it is written
     auto dst = [&](int c) -> double * {
       return (p.slices > 1 && p.part_stride == 0)
@@ -652,103 +479,6 @@ k_spectrum(const KParams p) {
         }
       };
 
-      // one step of the recurrence sweep for the thread's first K omegas: the
-      // base phase in FP64, then each omega by rotation.  MASK 0: no masking
-      // (tiles where no step cuts the block's omega range); 1: the step is
-      // skipped when the whole block is above its threshold and each omega is
-      // masked otherwise; 2: only the K-th omega is masked (sorted tiles, where
-      // the runs below the step's last kept run keep all their omegas).
-      // rec_acc: the accumulations of one step from its base sin/cos
-      // The second omega comes from the first by one complex multiplication;
-      // the third and fourth by the three-term recurrence z_{k+1} = 2 cos(d)
-      // z_k - z_{k-1} of equally spaced angles (two FMAs instead of two
-      // multiplications and two FMAs; over two terms its error growth is
-      // that of the multiplication's within a factor 3)
-      auto rec_acc = [&](auto Kc, auto Mc, float sn, float cn, double thr, float er, float ei,
-                         const float *a) {
-        constexpr int K = decltype(Kc)::value;
-        constexpr int MASK = decltype(Mc)::value;
-        float cp = 0.f, sp = 0.f;   // z_{k-1}
-        const float c2 = (SR_REC_CHEB && K >= 3) ? er + er : 0.f;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-          float cm = cn, sm = sn;
-          if (MASK == 1 || (MASK == 2 && k == K - 1)) {
-            const bool act = fabs(om_rev[k]) < thr;
-            cm = act ? cn : 0.f;
-            sm = act ? sn : 0.f;
-          }
-          split_acc<MODE, NA>(ps[k], a, cm, sm);
-          if (k + 1 < K) {
-            float cn2, sn2;
-            if (SR_REC_CHEB && k >= 1) {
-              cn2 = __builtin_fmaf(c2, cn, -cp);
-              sn2 = __builtin_fmaf(c2, sn, -sp);
-            } else {
-              cn2 = __builtin_fmaf(cn, er, -sn * ei);
-              sn2 = __builtin_fmaf(cn, ei, sn * er);
-            }
-            cp = cn;
-            sp = sn;
-            cn = cn2;
-            sn = sn2;
-          }
-        }
-      };
-      auto rec_step = [&](auto Kc, auto Mc, double tau, double thr, float er, float ei, const float *a) {
-        if (decltype(Mc)::value == 1 && thr <= w_lo) return;   // every omega of the block filtered out
-        float sn, cn;
-        sincos_rev(om0_rev * tau, &sn, &cn);
-        rec_acc(Kc, Mc, sn, cn, thr, er, ei, a);
-      };
-      // staged step jj of the recurrence sweep: two (far) or three (near)
-      // 16-byte reads of its record
-      auto rec_load = [&](int jj, double &tau, double &thr, float &er, float &ei, float *a) {
-        const RecStep<NA> &r = s_rec[jj];
-        const double2 tt = *(const double2 *)&r.tau;
-        const float4 u = *(const float4 *)&r.er;
-        tau = tt.x;
-        thr = tt.y;
-        er = u.x;
-        ei = u.y;
-        a[0] = u.z;
-        a[1] = u.w;
-        if constexpr (NA > 2) {
-          const float4 w = *(const float4 *)&r.amp[2];
-          a[2] = w.x;
-          a[3] = w.y;
-          a[4] = w.z;
-          a[5] = w.w;
-        }
-      };
-      // steps [j, jend) of the staged tile: groups of 4, then the tail
-      auto rec_sweep = [&](auto Kc, auto Mc, int &j, int jend) {
-        for (; j + 4 <= jend; j += 4) {
-          double tq[4], hq[4];
-          float erq[4], eiq[4], aq[4][NA];
-#pragma unroll
-          for (int q = 0; q < 4; q++) rec_load(j + q, tq[q], hq[q], erq[q], eiq[q], aq[q]);
-          if (SR_REC_PIPE && decltype(Mc)::value != 1) {
-            // the four base phases and sin/cos first (independent chains), then
-            // the accumulations
-            float sn[4], cn[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) sincos_rev(om0_rev * tq[q], &sn[q], &cn[q]);
-#pragma unroll
-            for (int q = 0; q < 4; q++) rec_acc(Kc, Mc, sn[q], cn[q], hq[q], erq[q], eiq[q], aq[q]);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 4; q++) rec_step(Kc, Mc, tq[q], hq[q], erq[q], eiq[q], aq[q]);
-          }
-        }
-        for (; j < jend; j++) {
-          double tau, thr;
-          float er, ei, a[NA];
-          rec_load(j, tau, thr, er, ei, a);
-          rec_step(Kc, Mc, tau, thr, er, ei, a);
-        }
-      };
-
       // one staged step of the direct sweeps; WIDE (FP64): the tile's phases
       // may reach the sin/cos table's limit
       auto direct_step = [&](int j, auto Wc) {
@@ -867,11 +597,7 @@ k_spectrum(const KParams p) {
       for (int64_t t0 = 0; t0 < n_act; t0 += T) {
         const int cnt = uni((int)min((int64_t)T, n_act - t0));
         __syncthreads();  // previous tile fully consumed
-        int step_on = 1;
         int st_wide = 0;
-        Amp st_amp[NA];
-        double st_tau = 0.0, st_thr = 0.0, st_prev = 0.0;
-        float st_rot[2] = {1.f, 0.f};
         if (tid < cnt) {
           // ---- stage: omega-independent part of step s = t0 + tid, in FP64 ----
           const int64_t s = t0 + tid;
@@ -882,9 +608,10 @@ k_spectrum(const KParams p) {
           const double gx = q.gx, gy = q.gy, gz = q.gz;
           const double thx = q.thx, thy = q.thy, thz = q.thz, phx = q.phx, phy = q.phy;
           double tau;
-          // tau_{s-1} (phase_{-1} = 0 at the first step): recomputed here by the
-          // tile's first thread, or by every thread without the exchange
-          const bool own_prev = kSplit && s > 0 && (!kExch || tid == 0);
+          Amp st_amp[NA];
+          // split: tau_{s-1} (phase_{-1} = 0 at the first step)
+          double st_prev = 0.0;
+          const bool own_prev = kSplit && s > 0;
           if (MODE == SR_MODE_FAR) {
             // kernel_farfield.cl:65-94
             tau = time - (xs * gx + ys * gy + zs * gz);
@@ -906,7 +633,7 @@ k_spectrum(const KParams p) {
             // split: the amplitude ends in FP32, so the hardware reciprocal
             // (relative error <= 4.6e-8 measured on gfx950) with one Newton
             // step (~1e-15) replaces the IEEE division
-            if (kSplit && SR_SPLIT_RCP) {
+            if (kSplit) {
               const double r = __builtin_amdgcn_rcp(c2);
               c2 = fma(r, fma(-c2, r, 1.0), r);
             } else {
@@ -947,160 +674,52 @@ k_spectrum(const KParams p) {
             st_amp[4] = (Amp)(r2 * ny);
             st_amp[5] = (Amp)(r2 * nz);
           }
-          st_tau = tau;
+          const int pos = late(tid);   // the staged slots' LDS addresses formed here
           if (kTab) st_wide = fabs(tau) * om_abs_max >= 0.5 * kTabMaxPhase;
-          if (kRec) sincos_rev(rot_rev * tau, &st_rot[1], &st_rot[0]);
-          if constexpr (kExch) s_rec[tid].tau = tau;   // in step order, for the next thread
-        }
-        if constexpr (kSplit) {
-          if (kExch) {
-            // every tau of the tile is in LDS; the staged copies are written
-            // after the step sort's barriers (or, unsorted, over the same value)
-            __syncthreads();
-            if (tid > 0 && tid < cnt) st_prev = s_rec[tid - 1].tau;
-          }
-          if (tid < cnt) {
+          if constexpr (kSplit) {
             // |omega tau_s - omega tau_{s-1}| < pi  <=>  |omega|/2pi < (1/2)/|tau_s - tau_{s-1}|
-            // (phase_{-1} = 0 at the first step); 1/0 gives +inf: always active
-            // (split: the hardware reciprocal with one Newton step, as for c2;
-            // the raw one, 4.6e-8, moved enough boundary decisions to raise the
-            // largest element error of the betatron spectrum from 1e-7 to 6e-7)
+            // (the hardware reciprocal with one Newton step, as for c2; the raw
+            // one, 4.6e-8, moved enough boundary decisions to raise the largest
+            // element error of the betatron spectrum from 1e-7 to 6e-7)
             // (d = 0: +inf, always active, as the division gives; the Newton
             // step alone would make it fma(-0, inf, 1) = NaN)
-            double thr;
-            if (SR_SPLIT_RCP) {
-              const double d = fabs(st_tau - st_prev);
-              const double r = __builtin_amdgcn_rcp(d);
-              thr = (d == 0.0) ? INFINITY : 0.5 * fma(r, fma(-d, r, 1.0), r);
-            } else {
-              thr = 0.5 / fabs(st_tau - st_prev);
-            }
-            st_thr = thr;
-            step_on = thr > w_hi;
+            const double d = fabs(tau - st_prev);
+            const double r = __builtin_amdgcn_rcp(d);
+            s_thr[pos] = (d == 0.0) ? INFINITY : 0.5 * fma(r, fma(-d, r, 1.0), r);
           }
-        }
-        // compaction (tiles without a snapshot record): bucket_s = number of runs
-        // that keep some omega at step s; a stable counting sort puts the steps
-        // in descending bucket order, so run r of rank rho sweeps exactly the
-        // first s_cntb[rho] steps.  Steps of bucket 0 are needed by no run.
-        const bool sort_tile = kCompact && rec_sortable && uni((cur.next >= 0 && cur.next < t0 + cnt) ? 0 : 1);
-        int pos = tid;
-        if (sort_tile) {
-          const int R = W * M;
-          int bucket = 0;
-          if (tid < cnt) {
-            if (SR_BUCKET_SEARCH) {
-              // R is a power of two; the count of sorted entries below thr
-              for (int h = R >> 1; h > 0; h >>= 1)
-                if (s_wsort[bucket + h - 1] < st_thr) bucket += h;
-              if (s_wsort[bucket] < st_thr) bucket++;
-            } else {
-              for (int r = 0; r < R; r++) bucket += (s_wmin[r] < st_thr) ? 1 : 0;
-            }
-          }
-          // per-wave counts in the order (bucket R..1) x (wave 0..W-1)
-          uint64_t mine = 0;
-          for (int b = 1; b <= R; b++) {
-            const uint64_t m = __ballot(bucket == b);
-            if (bucket == b) mine = m;
-            if (lane == 0) s_hist[(R - b) * W + wv] = __popcll(m);
-          }
-          __syncthreads();
-          if (wv == 0) {
-            const int n_ent = R * W;   // <= 64: one entry per lane
-            const int v = lane < n_ent ? s_hist[lane] : 0;
-            int inc = v;
-            for (int o = 1; o < kWave; o <<= 1) {
-              const int y = __shfl_up(inc, o);
-              if (lane >= o) inc += y;
-            }
-            if (lane < n_ent) s_off[lane] = inc - v;
-            // steps with bucket > b = everything before entry (b, wave 0)
-            if (lane < n_ent && lane % W == 0) s_cntb[R - lane / W] = inc - v;
-            if (lane == n_ent - 1) s_cntb[0] = inc;
-          }
-          __syncthreads();
-          const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
-          pos = (bucket > 0) ? s_off[(R - bucket) * W + wv] + __popcll(mine & below) : -1;
-        }
-        if (tid < cnt && pos >= 0) {
-          pos = late(pos);   // the staged slots' LDS addresses formed here
-          if constexpr (kRec) {
-            RecStep<NA> &r = s_rec[pos];
-            *(double2 *)&r.tau = make_double2(st_tau, st_thr);
-            *(float4 *)&r.er = make_float4(st_rot[0], st_rot[1], (float)st_amp[0], (float)st_amp[1]);
-            if constexpr (NA > 2)
-              *(float4 *)&r.amp[2] = make_float4((float)st_amp[2], (float)st_amp[3], (float)st_amp[4], (float)st_amp[5]);
-          } else {
-            s_tau[pos] = st_tau;
-            if (kSplit) s_thr[pos] = st_thr;
+          s_tau[pos] = tau;
 #pragma unroll
-            for (int c = 0; c < NA; c++) s_amp[c][pos] = st_amp[c];
-          }
+          for (int c = 0; c < NA; c++) s_amp[c][pos] = st_amp[c];
         }
-        // rec: the tile needs no masking when every step keeps the whole block.
-        // The block votes through one ballot per wave and an LDS word per wave
-        // (the block is one-dimensional: unlike the library's work-group
-        // reductions this keeps no y/z work-item ids alive, which cost the FP64
-        // near-field variant two spilled registers)
-        bool tile_on = false;
-        if constexpr (kRec || kTab) {
-          const bool pred = kRec ? (step_on == 0) : (st_wide != 0);   // rec: any step not keeping all
-          const uint64_t b = __ballot(pred);
+        // FP64: a vote through one ballot per wave and an LDS word per wave (the
+        // block is one-dimensional: unlike the library's work-group reductions
+        // this keeps no y/z work-item ids alive, which cost the near-field
+        // variant two spilled registers)
+        if constexpr (kTab) {
+          const uint64_t b = __ballot(st_wide != 0);
           if (lane == 0) s_vote[wv] = (b != 0) ? 1 : 0;
           __syncthreads();
           int any = 0;
           for (int w = 0; w < W; w++) any |= s_vote[w];
-          if constexpr (kRec)
-            tile_on = uni(any) == 0;
-          else
-            tile_wide = uni(any) != 0;
+          tile_wide = uni(any) != 0;
         } else {
           __syncthreads();
         }
 
         // ---- sweep, split at snapshot records falling inside the tile ----
-        if (sort_tile) {
-          // run k of this wave (rank s_rank[k*W + wave]) needs the first ck[k]
-          // steps; the runs ascend, so ck[0] >= ck[1] >= ... and the steps
-          // [ck[K], ck[K-1]) keep exactly the runs k < K (ck[M] = 0)
-          int ck[M];
-#pragma unroll
-          for (int k = 0; k < M; k++) ck[k] = uni(s_cntb[s_rank[k * W + vw]]);
-          int j = 0;
-          if (tile_on) {
-            // every valid omega of the block kept at every step: the wave's
-            // valid runs all have ck = cnt, runs past n_omega have ck = 0
-            rec_sweep(IC<M>(), IC<0>(), j, ck[0]);
-          } else {
-            rec_sweep(IC<M>(), IC<2>(), j, ck[M - 1]);
-            if (M >= 2) rec_sweep(IC<(M >= 2 ? M - 1 : 1)>(), IC<2>(), j, ck[M >= 2 ? M - 2 : 0]);
-            if (M >= 3) rec_sweep(IC<(M >= 3 ? M - 2 : 1)>(), IC<2>(), j, ck[M >= 3 ? M - 3 : 0]);
-            if (M >= 4) rec_sweep(IC<(M >= 4 ? M - 3 : 1)>(), IC<2>(), j, ck[0]);
-          }
+        int j = 0;
+        while (j < cnt) {
+          const bool rec_here = (cur.next >= 0) && (cur.next < t0 + cnt);
+          // records are strictly increasing, so cur.next >= t0 + j; the max()
+          // only guarantees forward progress
+          const int jend = uni(rec_here ? max(j + 1, (int)(cur.next - t0) + 1) : cnt);
+          direct_sweep(j, jend);
           kahan_fold();
-        } else {
-          int j = 0;
-          while (j < cnt) {
-            const bool rec_here = (cur.next >= 0) && (cur.next < t0 + cnt);
-            // records are strictly increasing, so cur.next >= t0 + j; the max()
-            // only guarantees forward progress
-            const int jend = uni(rec_here ? max(j + 1, (int)(cur.next - t0) + 1) : cnt);
-            if (kRec) {
-              if (tile_on)
-                rec_sweep(IC<M>(), IC<0>(), j, jend);
-              else
-                rec_sweep(IC<M>(), IC<1>(), j, jend);
-            } else {
-              direct_sweep(j, jend);
-            }
-            kahan_fold();
-            if (rec_here) {
-              emit(cur.slot);
-              const int64_t last = cur.next;
-              cur.slot++;
-              cur.advance(pt, p.n_snaps, last);
-            }
+          if (rec_here) {
+            emit(cur.slot);
+            const int64_t last = cur.next;
+            cur.slot++;
+            cur.advance(pt, p.n_snaps, last);
           }
         }
       }
@@ -1312,16 +931,26 @@ struct Plan {
   int sweep;     // SWEEP_*
   int waves;     // waves per block
   int M;         // omegas per thread
+  int groups;    // recurrence: groups of 32 omegas per tile (factored.h)
   int slices;
   int64_t blocks;
 };
 
-// omegas per thread each variant is built for (the near-field recurrence
-// keeps twice the far field's accumulators, so it stops at 2)
-int allowed_m(int mode, int prec, int sweep, int m) {
+// omegas per thread each direct variant is built for
+int allowed_m(int mode, int prec, int m) {
   if (prec == SR_PREC_F64) return m == 1 || m == 2;
-  if (sweep == SWEEP_REC) return mode == SR_MODE_FAR ? (m == 2 || m == 4) : m == 2;
   return m == 1 || m == 2 || (mode == SR_MODE_FAR && m == 4);
+}
+
+// vector instructions per step of a factored tile: the stage and the factors
+double factored_cost(bool far, int groups) {
+  if (far) return 2.5 + (groups == 4 ? 4.75 : groups == 8 ? 5.5 : 7.5);
+  return 9.75;
+}
+
+// omegas of one tile
+int64_t tile_run(const Plan &pl) {
+  return pl.sweep == SWEEP_REC ? 32 * (int64_t)pl.groups : (int64_t)kWave * pl.waves * pl.M;
 }
 
 // Tile shape: prefer the largest omega run per block (T*M) that is mostly
@@ -1331,50 +960,74 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   Plan pl;
   const int64_t n_om = g.n_omega;
   const int64_t n_dir = (int64_t)g.n_theta * g.n_phi;
-  // AUTO: the recurrence sweep for split spectra on linear grids (measured
-  // fastest there, far and near), the direct sweep otherwise
+  // AUTO: the factored tiles for split spectra on linear grids, except far-field
+  // grids of at most one 64-omega wave: there the direct sweep's sine per omega
+  // costs no more than forming the factors (32 betatron electrons on 64 x 32 x 32:
+  // 3.38 ms against 3.62; on 72 omegas 6.8 against 3.6)
   pl.sweep = SWEEP_DIRECT;
   if (o.precision == SR_PREC_SPLIT && g.omega_step != 0.0 &&
-      (o.sweep == SR_SWEEP_RECURRENCE || o.sweep == SR_SWEEP_AUTO))
+      (o.sweep == SR_SWEEP_RECURRENCE ||
+       (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave))))
     pl.sweep = SWEEP_REC;
-  int best_w = 1, best_m = 1;
-  double best_score = -1;
-  const int m_opts[3] = {1, 2, 4};
-  for (int w = 1; w <= 4; w *= 2) {
-    for (int mi = 0; mi < 3; mi++) {
-      const int m = m_opts[mi];
-      if (!allowed_m(g.mode, o.precision, pl.sweep, m)) continue;
-      const int64_t run = (int64_t)kWave * w * m;
-      const int64_t chunks = (n_om + run - 1) / run;
-      const double eff = (double)n_om / (double)(chunks * run);
-      if (eff < 0.75) continue;
-      // far-field recurrence: 4 omegas per thread in 2-wave blocks (one
-      // 512-omega chunk per direction, 3 waves per SIMD; when chosen: 5934 G
-      // evals/s on the betatron beam against 5267 for 2 omegas x 2 waves and
-      // 4871 for 2 x 4); elsewhere M = 2 measured fastest.  Blocks
-      // of 2 waves: with the tiles launched heaviest first, the finer tiles
-      // balance better (+8 % over 4 waves)
-      const bool rec_far = pl.sweep == SWEEP_REC && g.mode == SR_MODE_FAR;
-      const double mpref = rec_far ? (m == 4 ? 0.04 : (m == 2 ? 0.02 : 0.0)) : ((m == 2) ? 0.02 : 0.0);
-      const double wpref = (pl.sweep == SWEEP_REC && g.mode == SR_MODE_FAR && w == 2) ? 0.03 : 0.0;
-      // launches too small to fill the GPU (one particle: no slices to add
-      // waves) prefer the plan with the most waves: 256 CUs hold ~8K waves
-      const double fill =
-          std::min(1.0, (double)(chunks * n_dir * w * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices)) /
-                            8192.0);
-      const double score = eff * fill + 0.01 * w + mpref + wpref;
-      if (score > best_score) { best_score = score; best_w = w; best_m = m; }
+  int64_t chunks;
+  if (pl.sweep == SWEEP_REC) {
+    // groups of 32 omegas per tile (factored.h): the number whose tiles cost
+    // least, a step of a tile costing kFactoredStage for its stage and the
+    // matrix factors of NG groups
+    const bool far = g.mode == SR_MODE_FAR;
+    pl.M = (far && o.omega_per_lane != 2 && o.omega_per_lane != 1) ? 4 : 2;
+    const int max_groups = pl.M == 4 ? 16 : far ? 8 : 4;
+    double best = INFINITY;
+    pl.groups = 4;
+    for (int ng = 4; ng <= max_groups; ng *= 2) {
+      const int64_t c = (n_om + 32 * ng - 1) / (32 * ng);
+      const double cost = (double)c * factored_cost(far, ng);
+      if (cost < best) {
+        best = cost;
+        pl.groups = ng;
+      }
     }
+    chunks = (n_om + 32 * pl.groups - 1) / (32 * pl.groups);
+    // waves of a block share a tile's steps.  One each, but two for 16 groups
+    // (betatron beam, 24 x 8000 steps on 512 x 32 x 32: 8.1 ms against 9.1; the
+    // near-field screen with 4 groups the other way, 6.9 against 7.6), and more
+    // where the tiles and particle slices leave the GPU short of waves (one
+    // undulator electron on 256 x 32 x 32: 71 us with two, 94 with one)
+    pl.waves = pl.groups == 16 ? 2 : 1;
+    while (pl.waves < 4 &&
+           chunks * n_dir * pl.waves * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices) < 2048)
+      pl.waves *= 2;
+    if (o.waves_per_block > 0) pl.waves = o.waves_per_block;
+  } else {
+    pl.groups = 0;
+    int best_w = 1, best_m = 1;
+    double best_score = -1;
+    const int m_opts[3] = {1, 2, 4};
+    for (int w = 1; w <= 4; w *= 2) {
+      for (int mi = 0; mi < 3; mi++) {
+        const int m = m_opts[mi];
+        if (!allowed_m(g.mode, o.precision, m)) continue;
+        const int64_t run = (int64_t)kWave * w * m;
+        const int64_t c = (n_om + run - 1) / run;
+        const double eff = (double)n_om / (double)(c * run);
+        if (eff < 0.75) continue;
+        // M = 2 measured fastest
+        const double mpref = (m == 2) ? 0.02 : 0.0;
+        // launches too small to fill the GPU (one particle: no slices to add
+        // waves) prefer the plan with the most waves: 256 CUs hold ~8K waves
+        const double fill =
+            std::min(1.0, (double)(c * n_dir * w * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices)) /
+                              8192.0);
+        const double score = eff * fill + 0.01 * w + mpref;
+        if (score > best_score) { best_score = score; best_w = w; best_m = m; }
+      }
+    }
+    pl.waves = o.waves_per_block > 0 ? o.waves_per_block : best_w;
+    pl.M = o.omega_per_lane > 0 ? o.omega_per_lane : best_m;
+    if (!allowed_m(g.mode, o.precision, pl.M)) pl.M = 1;
+    const int64_t run = (int64_t)kWave * pl.waves * pl.M;
+    chunks = (n_om + run - 1) / run;
   }
-  if (best_score < 0) {
-    best_w = 1;
-    best_m = (pl.sweep == SWEEP_REC) ? 2 : 1;
-  }
-  pl.waves = o.waves_per_block > 0 ? o.waves_per_block : best_w;
-  pl.M = o.omega_per_lane > 0 ? o.omega_per_lane : best_m;
-  if (!allowed_m(g.mode, o.precision, pl.sweep, pl.M)) pl.M = (pl.sweep == SWEEP_REC) ? 2 : 1;
-  const int64_t run = (int64_t)kWave * pl.waves * pl.M;
-  const int64_t chunks = (n_om + run - 1) / run;
   const int64_t base_waves = chunks * n_dir * pl.waves;
   int s = 1;
   if (o.slices > 0) {
@@ -1389,7 +1042,12 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
     const double evals = (double)n_points * (double)(n_om * n_dir);
     const bool far_ordered = g.mode == SR_MODE_FAR && o.tile_order == 0;
     const bool big = evals >= kOrderSliceEvals && (g.mode != SR_MODE_FAR || far_ordered);
-    const int64_t target = big ? 64 * 1024 : 8 * 1024;
+    // factored tiles: ~32K waves from 1e10 evaluations on (24 x 4000 steps and
+    // more), where the finer tiles' shorter tail outweighs summing the slices:
+    // 48 electrons on the near-field screen 19.5 ms against 20.4 at 8K, 256 on
+    // 128 x 32 x 32 24.2 against 29.0
+    const bool fine = pl.sweep == SWEEP_REC && evals >= kOrderMinEvals;
+    const int64_t target = big ? 64 * 1024 : fine ? 32 * 1024 : 8 * 1024;
     auto orderable = [&](int64_t tiles) {
       return tiles <= kOrderMaxTiles && evals >= kOrderEvalsPerTile2 * (double)tiles * (double)tiles;
     };
@@ -1404,17 +1062,27 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   return pl;
 }
 
-template <int MODE, int PREC, int SWEEP, int M>
+template <int MODE, int PREC, int M>
 hipError_t launch_t(const KParams &kp, int64_t grid, int threads, hipStream_t st) {
-  const size_t lds = stage_lds_bytes<MODE, PREC, SWEEP>(threads) +
+  const size_t lds = stage_lds_bytes<MODE, PREC>(threads) +
                      ((PREC == SR_PREC_SPLIT) ? kahan_lds_bytes<MODE, M>(threads) : 0) +
                      (kp.acc_lds ? acc_lds_bytes<M>(threads) : 0);
   if (kp.pre)
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, SWEEP, M, true>), dim3((unsigned)grid), dim3(threads), lds, st,
+    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, true>), dim3((unsigned)grid), dim3(threads), lds, st,
                        kp);
   else
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, SWEEP, M, false>), dim3((unsigned)grid), dim3(threads), lds, st,
+    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, false>), dim3((unsigned)grid), dim3(threads), lds, st,
                        kp);
+  return hipGetLastError();
+}
+
+template <int MODE, int NG>
+hipError_t launch_factored(const KParams &kp, int64_t grid, int threads, hipStream_t st) {
+  const size_t lds = factored_lds<MODE, NG>(threads / kWave, kp.acc_lds != 0);
+  if (kp.pre)
+    hipLaunchKernelGGL((k_factored<MODE, NG, true>), dim3((unsigned)grid), dim3(threads), lds, st, kp);
+  else
+    hipLaunchKernelGGL((k_factored<MODE, NG, false>), dim3((unsigned)grid), dim3(threads), lds, st, kp);
   return hipGetLastError();
 }
 
@@ -1422,18 +1090,19 @@ template <int MODE>
 hipError_t launch_mode(const Plan &pl, int prec, const KParams &kp, int64_t grid, int threads,
                        hipStream_t st) {
   if (prec == SR_PREC_F64) {
-    if (pl.M == 2) return launch_t<MODE, SR_PREC_F64, SWEEP_DIRECT, 2>(kp, grid, threads, st);
-    return launch_t<MODE, SR_PREC_F64, SWEEP_DIRECT, 1>(kp, grid, threads, st);
+    if (pl.M == 2) return launch_t<MODE, SR_PREC_F64, 2>(kp, grid, threads, st);
+    return launch_t<MODE, SR_PREC_F64, 1>(kp, grid, threads, st);
   }
   if (pl.sweep == SWEEP_REC) {
-    if (MODE == SR_MODE_NEAR || pl.M == 2)
-      return launch_t<MODE, SR_PREC_SPLIT, SWEEP_REC, 2>(kp, grid, threads, st);
-    return launch_t<MODE, SR_PREC_SPLIT, SWEEP_REC, (MODE == SR_MODE_FAR ? 4 : 2)>(kp, grid, threads, st);
+    if (pl.groups == 4) return launch_factored<MODE, 4>(kp, grid, threads, st);
+    if (MODE == SR_MODE_FAR && pl.groups == 16)
+      return launch_factored<MODE, (MODE == SR_MODE_FAR ? 16 : 4)>(kp, grid, threads, st);
+    return launch_factored<MODE, (MODE == SR_MODE_FAR ? 8 : 4)>(kp, grid, threads, st);
   }
   if (MODE == SR_MODE_FAR && pl.M == 4)
-    return launch_t<MODE, SR_PREC_SPLIT, SWEEP_DIRECT, (MODE == SR_MODE_FAR ? 4 : 2)>(kp, grid, threads, st);
-  if (pl.M == 2) return launch_t<MODE, SR_PREC_SPLIT, SWEEP_DIRECT, 2>(kp, grid, threads, st);
-  return launch_t<MODE, SR_PREC_SPLIT, SWEEP_DIRECT, 1>(kp, grid, threads, st);
+    return launch_t<MODE, SR_PREC_SPLIT, (MODE == SR_MODE_FAR ? 4 : 2)>(kp, grid, threads, st);
+  if (pl.M == 2) return launch_t<MODE, SR_PREC_SPLIT, 2>(kp, grid, threads, st);
+  return launch_t<MODE, SR_PREC_SPLIT, 1>(kp, grid, threads, st);
 }
 
 int check_grid(const sr_grid *g) {
@@ -1548,7 +1217,7 @@ size_t order_bytes(const Plan &pl, const sr_grid &g, const sr_opts &o, int64_t n
 int run(KParams &kp, const Plan &pl, const sr_grid &g, const sr_opts &o, void *ws, size_t ws_bytes,
         hipStream_t st, bool want_pre = false, size_t need_order = 0) {
   const int threads = kWave * pl.waves;
-  const int64_t run = (int64_t)threads * pl.M;
+  const int64_t run = tile_run(pl);
   kp.n_chunks = (uint32_t)((g.n_omega + run - 1) / run);
   kp.slices = pl.slices;
   kp.n_tiles = pl.blocks;

@@ -1,0 +1,120 @@
+"""The split-precision spectrum on linear omega grids (matrix products over the
+steps, synchrad_amd/csrc/factored.h) against the CPU FP64 oracle, at the sizes
+where it can go wrong: omega counts around the 32-omega groups and the 128-,
+256- and 512-omega tiles, step counts around the 63-step stretches and the
+32-step products, every order of the omegas (descending, negative, through
+zero), and tracks whose amplitude jumps or vanishes.
+
+Bound, per complex field component: each term A_s e^{i phase} passes through at
+most eleven FP32-level roundings (two phasor factors and their product on each
+side, the amplitude, two fp16 two-word splits of 2^-22 and the dropped low-low
+product of 2^-22), at most 11 * 2^-22 = 2.6e-6 of |A_s| in all, and the FP32
+accumulation of up to 256 steps (24 additions of 2^-24 of the partial sum) adds
+1.4e-6 of the sum of |A_s|: 4e-6 of it together.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle
+from synchrad_amd import engine, workloads
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 4e-6
+
+
+def _far_abs_sum(track, axes, dt):
+    """dt * sum_s |A_s| per direction, (n_theta, n_phi), from the reference's definition."""
+    x, y, z, ux, uy, uz = track[:6]
+    b = np.stack([ux, uy, uz], 1) / np.sqrt(1 + ux ** 2 + uy ** 2 + uz ** 2)[:, None]
+    a, m = np.diff(b, axis=0) / dt, 0.5 * (b[1:] + b[:-1])
+    out = np.zeros((axes["theta"].size, axes["phi"].size))
+    for i, th in enumerate(axes["theta"]):
+        for j, ph in enumerate(axes["phi"]):
+            n = np.array([np.sin(th) * np.cos(ph), np.sin(th) * np.sin(ph), np.cos(th)])
+            c2 = 1 / (1 - m @ n)
+            c1 = (a @ n) * c2 ** 2
+            out[i, j] = dt * np.linalg.norm(c1[:, None] * (n - m) - c2[:, None] * a, axis=1).sum()
+    return out
+
+
+def _run(mode, comp, tracks, axes, dt, tuning=None, L_screen=None, **kw):
+    batch = engine.DeviceBatch(engine.pack_tracks(tracks, dt=dt, **kw))
+    ax1 = axes["theta"] if mode == "far" else axes["radius"]
+    grid = engine.DeviceGrid(mode, axes["omega"], ax1, axes["phi"], L_screen=L_screen)
+    assert grid.omega_step != 0.0
+    outs = engine.spectrum(batch, grid, comp=comp, precision="float", tuning=tuning)
+    torch.cuda.synchronize()
+    return {k: o.cpu().numpy().swapaxes(-1, -3) for k, o in zip(engine.COMP_KEYS[comp], outs)}
+
+
+def _omegas(kind, n):
+    lo, hi = 1.0 * workloads.KEV_PER_INV_M, 75.0 * workloads.KEV_PER_INV_M
+    return {"up": np.linspace(lo, hi, n), "down": np.linspace(hi, lo, n), "negative": np.linspace(-hi, -lo, n),
+            "cross": np.linspace(-0.4 * hi, hi, n), "cross down": np.linspace(0.6 * hi, -hi, n)}[kind]
+
+
+CASES = [("up", n, 200, 0, 0) for n in (2, 31, 33, 127, 128, 129, 256, 300, 512, 513, 700)] + \
+        [("up", 96, n, 0, w) for n, w in ((2, 1), (33, 1), (63, 1), (64, 2), (65, 4), (127, 2), (700, 4))] + \
+        [(kind, n, 300, m, 0) for kind, n, m in (("down", 200, 0), ("negative", 150, 2), ("cross", 257, 0),
+                                                  ("cross down", 520, 4))]
+
+
+@pytest.mark.parametrize("kind,n_omega,n_steps,M,W", CASES)
+def test_far_edges(kind, n_omega, n_steps, M, W):
+    wl = workloads.config2(n_particles=1, n_steps=n_steps, grid=(8, 4, 3))
+    axes = dict(wl.axes, omega=_omegas(kind, n_omega))
+    tr, dt = wl.track_list(), wl.batch.dt
+    ref = oracle.spectrum("far", "cartesian_complex", tr, axes, dt)
+    got = _run("far", "cartesian_complex", tr, axes, dt, engine.Tuning(omega_per_lane=M, waves_per_block=W))
+    scale = _far_abs_sum(tr[0], axes, dt)[None, None]
+    worst = max(float(np.max(np.abs(got[k] - ref[k]) / scale)) for k in ref)
+    print(f"{kind} {n_omega} omegas {n_steps} steps M={M} W={W}: {worst:.2e} of sum |A|", flush=True)
+    assert worst <= BOUND
+
+
+@pytest.mark.parametrize("n_omega,n_steps", [(64, 65), (130, 500), (300, 127)])
+def test_near_edges(n_omega, n_steps):
+    wl = workloads.config4(n_particles=1)
+    tr = [[c[:n_steps] for c in wl.track_list()[0][:6]] + [1.0, 0]]
+    axes = {"omega": np.linspace(wl.axes["omega"][0], wl.axes["omega"][-1], n_omega),
+            "radius": np.linspace(0.0, 0.07, 3), "phi": np.array([0.0, 2.0])}
+    dt, L = wl.batch.dt, wl.L_screen
+    ref = oracle.spectrum("near", "cartesian_complex", tr, axes, dt, L_screen=L)
+    got = _run("near", "cartesian_complex", tr, axes, dt, L_screen=L)
+    # |v2| + omega |v1| summed over the steps at each screen point
+    x, y, z, ux, uy, uz = tr[0][:6]
+    b = (np.stack([ux, uy, uz], 1) / np.sqrt(1 + ux ** 2 + uy ** 2 + uz ** 2)[:, None])[:-1]
+    om = 2 * np.pi * axes["omega"]
+    for i, r in enumerate(axes["radius"]):
+        for j, ph in enumerate(axes["phi"]):
+            d = np.array([r * np.cos(ph), r * np.sin(ph), L]) - np.stack([x, y, z], 1)[:-1]
+            R = np.linalg.norm(d, axis=1)
+            n = d / R[:, None]
+            total = dt * ((1 / R ** 2).sum() + om * (np.linalg.norm(b - n, axis=1) / R).sum())
+            for k in ref:
+                assert np.max(np.abs(got[k] - ref[k])[0, :, i, j] / total) <= BOUND, (k, i, j)
+
+
+def test_amplitude_range_and_snapshots():
+    """An amplitude that is zero for most of the track, tiny, then 1e6 times
+    larger: the scale of the fp16 words follows it, and the snapshots taken
+    before and after keep their own accuracy (relative to the sum so far)."""
+    n, dt = 600, 2e-4
+    s = np.arange(n) * dt
+    kick = np.where(np.arange(n) < 200, 0.0, np.where(np.arange(n) < 400, 1e-6, 1.0))
+    ux = kick * np.sin(40 * s)
+    gamma = 30.0
+    uz = np.sqrt(gamma ** 2 - 1 - ux ** 2)
+    x = np.cumsum(ux / gamma) * dt
+    z = np.cumsum(uz / gamma) * dt
+    tr = [[x, np.zeros(n), z, ux, np.zeros(n), uz, 1.0, 0]]
+    axes = {"omega": np.linspace(10.0, 800.0, 100), "theta": np.linspace(0.0, 0.03, 3), "phi": np.array([0.3, 2.0])}
+    ref = oracle.spectrum("far", "cartesian_complex", tr, axes, dt, it_range=(0, n), nSnaps=3)
+    got = _run("far", "cartesian_complex", tr, axes, dt, it_range=(0, n), nSnaps=3)
+    for snap, end in enumerate((200, 400, 600)):
+        scale = _far_abs_sum([c[:end] for c in tr[0][:6]], axes, dt)[None] + 1e-300
+        for k in ref:
+            assert np.isfinite(got[k]).all()
+            assert np.max(np.abs(got[k][snap] - ref[k][snap]) / scale) <= BOUND, (k, snap)
