@@ -118,3 +118,26 @@ def test_amplitude_range_and_snapshots():
         for k in ref:
             assert np.isfinite(got[k]).all()
             assert np.max(np.abs(got[k][snap] - ref[k][snap]) / scale) <= BOUND, (k, snap)
+
+
+def test_small_component_keeps_its_accuracy():
+    """A vertical motion 1e-7 of the horizontal one: each amplitude word has its
+    own scale, so the phi component is as accurate, relative to its own sum, as
+    the theta component (one common scale would leave it 1e-3 off)."""
+    wl = workloads.config1()
+    x, y, z, ux, uy, uz = wl.track_list()[0][:6]
+    n, dt = 700, wl.batch.dt
+    uy = 1e-7 * np.roll(ux, 9)
+    y = np.cumsum(uy / 100.0) * dt
+    tr = [[c[:n] for c in (x, y, z, ux, uy, uz)] + [1.0, 0]]
+    axes = dict(wl.axes, omega=np.linspace(wl.axes["omega"][0], wl.axes["omega"][-1], 100),
+                theta=np.linspace(0.0, 0.01, 3), phi=np.array([0.0]))
+    ref = oracle.spectrum("far", "spheric_complex", tr, axes, dt)
+    got = _run("far", "spheric_complex", tr, axes, dt)
+    for pair in (("thetare", "thetaim"), ("phire", "phiim")):
+        err = np.sqrt(sum(np.sum((got[k] - ref[k]) ** 2) for k in pair))
+        size = np.sqrt(sum(np.sum(ref[k] ** 2) for k in pair))
+        print(f"{pair[0][:-2]}: size {size:.2e} rel-L2 {err / size:.2e}", flush=True)
+        # BOUND is relative to sum |A_s|; on the undulator line the sum itself is
+        # at least a tenth of it in the 2-norm over these omegas
+        assert err <= 10 * BOUND * size
