@@ -530,7 +530,7 @@ size_t adjoint_ws(const sr_tracks &t, const sr_grid &g, const APlan &pl, bool ow
   const size_t n_grid = (size_t)g.n_omega * g.n_theta * g.n_phi;
   return (adjoint_slab_words(t, pl) + (own_fields ? 6 * (size_t)pl.chunk * n_grid : 0) +
           6 * (size_t)t.n_points) * sizeof(double) +
-         (own_fields ? fields_order_space(g, precision, pl.chunk) : 0);
+         (own_fields ? fields_order_space(t, g, precision, pl.chunk) : 0);
 }
 
 // the adjoint; fields_in = NULL: the fields are computed chunk by chunk in the
@@ -577,7 +577,7 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
   double *fields = (double *)workspace + adjoint_slab_words(*t, pl);
   double *pre = own ? fields + 6 * (size_t)pl.chunk * (size_t)p.n_grid : fields;
   void *order_ws = own ? (void *)(pre + 6 * (size_t)t->n_points) : nullptr;
-  const size_t order_space = own ? fields_order_space(*g, o->precision, pl.chunk) : 0;
+  const size_t order_space = own ? fields_order_space(*t, *g, o->precision, pl.chunk) : 0;
   p.F = own ? fields : fields_in;
   p.pre = pre;
   hipStream_t st = (hipStream_t)stream;
@@ -638,7 +638,7 @@ int sr_far_fields_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid, 
   int rc = adjoint_check(tracks, grid, opts);
   if (rc) return rc;
   *bytes = 6 * (size_t)tracks->n_points * sizeof(double) +
-           fields_order_space(*grid, opts->precision, tracks->n_particles);
+           fields_order_space(*tracks, *grid, opts->precision, tracks->n_particles);
   return SR_OK;
 }
 
@@ -652,7 +652,7 @@ int sr_far_fields_batch(const sr_tracks *t, const sr_grid *g, const sr_opts *o, 
   if (outs)
     for (int c = 0; c < n_out; c++)
       if (!outs[c]) return fail(SR_ERR_INVALID, "outs[%d] is NULL", c);
-  const size_t order_space = fields_order_space(*g, o->precision, t->n_particles);
+  const size_t order_space = fields_order_space(*t, *g, o->precision, t->n_particles);
   const size_t need = 6 * (size_t)t->n_points * sizeof(double) + order_space;
   if (!workspace || workspace_bytes < need)
     return fail(SR_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);

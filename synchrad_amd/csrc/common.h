@@ -13,6 +13,7 @@ namespace sr {
 
 constexpr int kWave = 64;
 constexpr int kMaxT = 256;        // threads per block = steps per LDS tile
+constexpr int kMaxParts = 16;     // waves per block of the FP64 tile kernel
 constexpr int kMaxSlices = 32;
 constexpr int kMaxOut = 6;
 
@@ -44,7 +45,7 @@ int spectrum_fields(const sr_tracks &t, const sr_grid &g, int32_t precision, int
                     const double *pre, double *F, hipStream_t st, void *order_ws = nullptr,
                     size_t order_ws_bytes = 0);
 // workspace for the tile order of a fields launch of n_particles particles
-size_t fields_order_space(const sr_grid &g, int32_t precision, int64_t n_particles);
+size_t fields_order_space(const sr_tracks &t, const sr_grid &g, int32_t precision, int64_t n_particles);
 
 // ---------------------------------------------------------------------------
 // device helpers

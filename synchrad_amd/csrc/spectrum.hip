@@ -224,7 +224,7 @@ struct WavesPerEU {
 // PRE: the step data come from the pre-pass records (batch calls); without
 // them (the per-particle and no-allocation calls) the stage forms them from u
 template <int MODE, int PREC, int M, bool PRE>
-__global__ void __launch_bounds__(kMaxT)
+__global__ void __launch_bounds__(PREC == SR_PREC_F64 ? kWave * kMaxParts : kMaxT)
 __attribute__((amdgpu_waves_per_eu(WavesPerEU<MODE, PREC, M>::value)))
 k_spectrum(const KParams p) {
   static_assert(PREC == SR_PREC_SPLIT || M <= 2, "the FP64 sweep holds one or two omegas per thread");
@@ -237,7 +237,7 @@ k_spectrum(const KParams p) {
   constexpr int NA = amp_words<MODE, PREC>();
   constexpr int NC = (MODE == SR_MODE_FAR) ? 2 * NA : 6;   // real accumulators per omega
   constexpr int NP = (MODE == SR_MODE_FAR) ? NC : 12;      // split register partials per omega
-  constexpr int kMaxW = kMaxT / kWave;                 // waves per block
+  constexpr int kMaxW = kSplit ? kMaxT / kWave : kMaxParts;   // waves per block
 
   extern __shared__ __align__(16) char s_dyn_raw[];
   // FP64 sin/cos table (sincos_table) and the largest |omega| of the grid
@@ -246,8 +246,12 @@ k_spectrum(const KParams p) {
   __shared__ double s_wmax[kTab ? kMaxW : 1];
   __shared__ int s_vote[kMaxW];   // per-wave votes of a block-wide any/all
 
-  const int T = blockDim.x;
-  const int tid = threadIdx.x;
+  // the block's groups of T threads (FP64; the split sweep has one) each hold the
+  // tile's omegas and sweep a part of every track; their sums meet at the records
+  const int P = kSplit ? 1 : p.parts;
+  const int T = kSplit ? (int)blockDim.x : (int)blockDim.x / P;
+  const int grp = kSplit ? 0 : uni((int)threadIdx.x / T);
+  const int tid = (int)threadIdx.x - grp * T;
   const int W = T / kWave;
   const int wv = uni(tid / kWave);   // wave-uniform: its derived indices stay scalar
   const int lane = tid % kWave;
@@ -255,28 +259,30 @@ k_spectrum(const KParams p) {
   // sin/cos table's wide-phase form
   double om_abs_max = 0.0;
   if (kTab) {
-    for (int i = tid; i < kSinCosTab; i += T) {
+    for (int i = threadIdx.x; i < kSinCosTab; i += blockDim.x) {
       double sv, cv;
       sincospi((double)i / (kSinCosTab / 2), &sv, &cv);
       s_sct[i] = make_double2(sv, cv);
     }
     double m = 0.0;
-    for (int64_t i = tid; i < (int64_t)p.n_omega; i += T) m = fmax(m, fabs(p.omega[i]));
+    for (int64_t i = threadIdx.x; i < (int64_t)p.n_omega; i += blockDim.x) m = fmax(m, fabs(p.omega[i]));
     for (int o = kWave / 2; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-    if (lane == 0) s_wmax[wv] = m;
+    if (lane == 0) s_wmax[grp * W + wv] = m;
     __syncthreads();
-    for (int w = 0; w < W; w++) om_abs_max = fmax(om_abs_max, s_wmax[w]);
+    for (int w = 0; w < P * W; w++) om_abs_max = fmax(om_abs_max, s_wmax[w]);
   }
-  // dynamic LDS: the staged tile (s_tau[T], s_thr[T] (split), s_amp[NA][T]), then
-  // the Kahan state, then the particle sums
-  double *const s_tau = (double *)s_dyn_raw;
+  // dynamic LDS: the groups' staged tiles (s_tau[T], s_thr[T] (split), s_amp[NA][T]),
+  // then the Kahan state (split), the particle sums, and the groups' sums of one
+  // amplitude word on their way to the first group
+  double *const s_tau = (double *)(s_dyn_raw + grp * stage_lds_bytes<MODE, PREC>(T));
   double *const s_thr = s_tau + T;
   const LdsRows<Amp> s_amp{(Amp *)(s_tau + (kSplit ? 2 : 1) * T), T};
-  float *const s_dyn = (float *)(s_dyn_raw + stage_lds_bytes<MODE, PREC>(T));
+  float *const s_dyn = (float *)(s_dyn_raw + P * stage_lds_bytes<MODE, PREC>(T));
   float *const s_ks = s_dyn + tid;                       // S[c*M+k] at s_ks[(c*M+k)*T]
   float *const s_kc = s_dyn + (size_t)NC * M * T + tid;  // C likewise
   // particle sums of the single output, k-th omega at s_acc[k*T]
   double *const s_acc = (double *)((char *)s_dyn + (kSplit ? kahan_lds_bytes<MODE, M>(T) : 0)) + tid;
+  double *const s_sum = s_acc + (p.acc_lds ? M * T : 0);   // [P - 1][M][T]
   const double dt = p.dt;
   const double dtInv = 1.0 / dt;
   const bool spheric = (p.comp == SR_COMP_SPHERIC || p.comp == SR_COMP_SPHERIC_COMPLEX);
@@ -358,7 +364,7 @@ k_spectrum(const KParams p) {
                  : p.out[c];
     };
 
-    if (late_s(p.acc_lds)) {
+    if (late_s(p.acc_lds) && grp == 0) {
 #pragma unroll
       for (int k = 0; k < M; k++) s_acc[k * T] = 0.0;
     }
@@ -594,8 +600,33 @@ k_spectrum(const KParams p) {
         }
       };
 
-      for (int64_t t0 = 0; t0 < n_act; t0 += T) {
-        const int cnt = uni((int)min((int64_t)T, n_act - t0));
+      // FP64: tau of one step, as the stage forms it
+      auto tau_at = [&](int64_t s) {
+        const int64_t gs = pt.off + s;
+        const double time = (double)(uint32_t)(pt.its + (uint32_t)s) * dt;
+        const Geom q = geom();
+        if (MODE == SR_MODE_FAR) return time - (p.x[gs] * q.gx + p.y[gs] * q.gy + p.z[gs] * q.gz);
+        const double rx = q.gx - p.x[gs], ry = q.gy - p.y[gs], rz = q.gz - p.z[gs];
+        return time + sqrt(rx * rx + ry * ry + rz * rz);
+      };
+
+      // the steps up to each snapshot record, [done, seg_hi), cut into the groups'
+      // parts of `per` steps; the records after the last active step (global
+      // it_range mode) see the final sums
+      int64_t done = 0;
+      while (cur.next >= 0) {
+      const int64_t seg_hi = max(done, min(cur.next + 1, n_act));
+      const int64_t per = (seg_hi - done + P - 1) / P;
+      const int64_t lo = min(done + grp * per, seg_hi), hi = min(lo + per, seg_hi);
+      if (!kSplit) {
+        // FP64: the phase before the part's first step (phase_{-1} = 0)
+        const double before = lo > 0 ? tau_at(lo - 1) : 0.0;
+#pragma unroll
+        for (int k = 0; k < M; k++) prev[k] = om[k] * before;
+      }
+      for (int64_t it = 0; it < per; it += T) {
+        const int64_t t0 = lo + it;
+        const int cnt = uni((int)max((int64_t)0, min((int64_t)T, hi - t0)));
         __syncthreads();  // previous tile fully consumed
         int st_wide = 0;
         if (tid < cnt) {
@@ -697,10 +728,10 @@ k_spectrum(const KParams p) {
         // variant two spilled registers)
         if constexpr (kTab) {
           const uint64_t b = __ballot(st_wide != 0);
-          if (lane == 0) s_vote[wv] = (b != 0) ? 1 : 0;
+          if (lane == 0) s_vote[grp * W + wv] = (b != 0) ? 1 : 0;
           __syncthreads();
           int any = 0;
-          for (int w = 0; w < W; w++) any |= s_vote[w];
+          for (int w = 0; w < W; w++) any |= s_vote[grp * W + w];
           tile_wide = uni(any) != 0;
         } else {
           __syncthreads();
@@ -708,30 +739,37 @@ k_spectrum(const KParams p) {
 
         // ---- sweep, split at snapshot records falling inside the tile ----
         int j = 0;
-        while (j < cnt) {
-          const bool rec_here = (cur.next >= 0) && (cur.next < t0 + cnt);
-          // records are strictly increasing, so cur.next >= t0 + j; the max()
-          // only guarantees forward progress
-          const int jend = uni(rec_here ? max(j + 1, (int)(cur.next - t0) + 1) : cnt);
-          direct_sweep(j, jend);
-          kahan_fold();
-          if (rec_here) {
-            emit(cur.slot);
-            const int64_t last = cur.next;
-            cur.slot++;
-            cur.advance(pt, p.n_snaps, last);
+        direct_sweep(j, cnt);
+        kahan_fold();
+      }
+      done = seg_hi;
+      if (!kSplit && P > 1) {
+        // the other groups' sums so far go to the first group, one word at a time
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+          __syncthreads();
+          if (grp > 0) {
+#pragma unroll
+            for (int k = 0; k < M; k++) {
+              s_sum[((grp - 1) * M + k) * T] = fs[k][c];
+              fs[k][c] = 0.0;
+            }
+          }
+          __syncthreads();
+          if (grp == 0) {
+            for (int q1 = 0; q1 < P - 1; q1++)
+#pragma unroll
+              for (int k = 0; k < M; k++) fs[k][c] += s_sum[(q1 * M + k) * T];
           }
         }
       }
-      // records after the last active step (global it_range mode) see the final sums
-      while (cur.next >= 0) {
-        emit(cur.slot);
-        const int64_t last = cur.next;
-        cur.slot++;
-        cur.advance(pt, p.n_snaps, last);
+      if (grp == 0) emit(cur.slot);
+      const int64_t last = cur.next;
+      cur.slot++;
+      cur.advance(pt, p.n_snaps, last);
       }
     }
-    if (late_s(p.acc_lds)) {
+    if (late_s(p.acc_lds) && grp == 0) {
 #pragma unroll 1
       for (int k = 0; k < M; k++) {
         const int wk = omega_slot(k);
@@ -932,6 +970,7 @@ struct Plan {
   int waves;     // waves per block
   int M;         // omegas per thread
   int groups;    // recurrence: groups of 32 omegas per tile (factored.h)
+  int parts;     // FP64: groups of threads that share a tile's steps
   int slices;
   int64_t blocks;
 };
@@ -953,10 +992,14 @@ int64_t tile_run(const Plan &pl) {
   return pl.sweep == SWEEP_REC ? 32 * (int64_t)pl.groups : (int64_t)kWave * pl.waves * pl.M;
 }
 
+int64_t mean_steps(const sr_tracks &t) { return t.n_particles > 0 ? t.n_points / t.n_particles : 0; }
+
 // Tile shape: prefer the largest omega run per block (T*M) that is mostly
 // used, then enough particle slices to put ~8 waves on each of the 1024 SIMDs.
-// n_points: samples of the batch (0: unknown), for the size of the launch
-Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t n_snaps, int64_t n_points = 0) {
+// n_points: samples of the batch (0: unknown), for the size of the launch;
+// mean_steps: per particle, for the groups that share a tile's steps
+Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t n_snaps, int64_t n_points,
+               int64_t mean_steps) {
   Plan pl;
   const int64_t n_om = g.n_omega;
   const int64_t n_dir = (int64_t)g.n_theta * g.n_phi;
@@ -969,6 +1012,12 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
       (o.sweep == SR_SWEEP_RECURRENCE ||
        (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave))))
     pl.sweep = SWEEP_REC;
+  // FP64: groups of threads that may share a tile's steps: blocks of at most
+  // kMaxParts waves, two staged tiles of steps for each
+  auto part_limit = [&](int w) -> int64_t {
+    if (o.precision != SR_PREC_F64) return 1;
+    return std::max<int64_t>(1, std::min<int64_t>(kMaxParts / w, mean_steps / (2 * kWave * w)));
+  };
   int64_t chunks;
   if (pl.sweep == SWEEP_REC) {
     // groups of 32 omegas per tile (factored.h): the number whose tiles cost
@@ -1011,13 +1060,14 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
         const int64_t c = (n_om + run - 1) / run;
         const double eff = (double)n_om / (double)(c * run);
         if (eff < 0.75) continue;
-        // M = 2 measured fastest
-        const double mpref = (m == 2) ? 0.02 : 0.0;
+        // M = 2 measured fastest, also against twice the waves (256 omegas FP64: one
+        // undulator electron 0.38 ms at 2 x 2 waves, 0.42 at 1 x 4)
+        const double mpref = (m == 2) ? 0.03 : 0.0;
         // launches too small to fill the GPU (one particle: no slices to add
         // waves) prefer the plan with the most waves: 256 CUs hold ~8K waves
-        const double fill =
-            std::min(1.0, (double)(c * n_dir * w * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices)) /
-                              8192.0);
+        const double fill = std::min(1.0, (double)(c * n_dir * w * part_limit(w) *
+                                                   std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices)) /
+                                              8192.0);
         const double score = eff * fill + 0.01 * w + mpref;
         if (score > best_score) { best_score = score; best_w = w; best_m = m; }
       }
@@ -1057,6 +1107,15 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   }
   if (s > n_particles) s = (int)std::max<int64_t>(1, n_particles);
   pl.slices = s;
+  // FP64: launches short of waves (a few particles on a few directions) let several
+  // groups of threads share each tile's steps, up to the 4K waves that run at once
+  // (powers of two, so that blocks of 2 to 16 waves fill a CU's 16).  One undulator
+  // electron, 1600 steps: on 32 x 4 x 4 46 us with the groups, 228 without; on
+  // 256 x 32 x 32 (2 groups) 646 us through the calculator against 679; the adjoint of
+  // 8 electrons on 100 x 12 x 12 674 us against 772.  From 4K waves on the launch is the
+  // same as without.
+  pl.parts = 1;
+  while (2 * pl.parts <= part_limit(pl.waves) && base_waves * s * pl.parts < 4096) pl.parts *= 2;
   pl.blocks = chunks * n_dir * s;
   (void)n_snaps;
   return pl;
@@ -1064,9 +1123,10 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
 
 template <int MODE, int PREC, int M>
 hipError_t launch_t(const KParams &kp, int64_t grid, int threads, hipStream_t st) {
-  const size_t lds = stage_lds_bytes<MODE, PREC>(threads) +
-                     ((PREC == SR_PREC_SPLIT) ? kahan_lds_bytes<MODE, M>(threads) : 0) +
-                     (kp.acc_lds ? acc_lds_bytes<M>(threads) : 0);
+  const int T = threads / kp.parts;
+  const size_t lds = kp.parts * stage_lds_bytes<MODE, PREC>(T) +
+                     ((PREC == SR_PREC_SPLIT) ? kahan_lds_bytes<MODE, M>(T) : 0) +
+                     (kp.acc_lds ? acc_lds_bytes<M>(T) : 0) + (kp.parts - 1) * acc_lds_bytes<M>(T);
   if (kp.pre)
     hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, true>), dim3((unsigned)grid), dim3(threads), lds, st,
                        kp);
@@ -1216,7 +1276,8 @@ size_t order_bytes(const Plan &pl, const sr_grid &g, const sr_opts &o, int64_t n
 // partial spectra, the step data, the tile costs and order.
 int run(KParams &kp, const Plan &pl, const sr_grid &g, const sr_opts &o, void *ws, size_t ws_bytes,
         hipStream_t st, bool want_pre = false, size_t need_order = 0) {
-  const int threads = kWave * pl.waves;
+  const int threads = kWave * pl.waves * pl.parts;
+  kp.parts = pl.parts;
   const int64_t run = tile_run(pl);
   kp.n_chunks = (uint32_t)((g.n_omega + run - 1) / run);
   kp.slices = pl.slices;
@@ -1329,7 +1390,7 @@ int single_particle(int32_t mode, int32_t comp, double *const *outs, const doubl
   kp.single_its = itStart;
   kp.single_ite = itEnd;
   fill_grid(kp, g, o, n_out, outs);
-  Plan pl = make_plan(g, o, 1, nSnaps);
+  Plan pl = make_plan(g, o, 1, nSnaps, nSteps, nSteps);
   pl.slices = 1;  // one particle: no slices, no workspace
   slice_particles(kp, 1, 1, nullptr);
   return run(kp, pl, g, o, nullptr, 0, (hipStream_t)stream);
@@ -1373,8 +1434,8 @@ sr_opts fields_opts(int32_t precision) {
 }
 }  // namespace
 
-size_t fields_order_space(const sr_grid &g, int32_t precision, int64_t n_particles) {
-  const Plan pl = make_plan(g, fields_opts(precision), std::max<int64_t>(n_particles, 1), 1);
+size_t fields_order_space(const sr_tracks &t, const sr_grid &g, int32_t precision, int64_t n_particles) {
+  const Plan pl = make_plan(g, fields_opts(precision), std::max<int64_t>(n_particles, 1), 1, 0, mean_steps(t));
   if (pl.blocks > kOrderMaxTiles) return 0;
   return ((size_t)pl.blocks * (sizeof(float) + sizeof(int32_t)) + 255) / 256 * 256;
 }
@@ -1400,7 +1461,7 @@ int spectrum_fields(const sr_tracks &t, const sr_grid &g, int32_t precision, int
   double *outs[kMaxOut];
   for (int c = 0; c < 6; c++) outs[c] = F + (int64_t)c * np * n_grid;
   fill_grid(kp, g, o, 6, outs);
-  const Plan pl = make_plan(g, o, np, 1);
+  const Plan pl = make_plan(g, o, np, 1, 0, mean_steps(t));
   for (int q = 0; q <= pl.slices; q++) kp.slice_lo[q] = p_begin + np * q / pl.slices;
   kp.part_base = p_begin;
   kp.part_stride = n_grid;
@@ -1434,7 +1495,7 @@ int sr_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid, const sr_op
   *bytes = 0;
   if ((rc = check_tracks(tracks)) || (rc = check_grid(grid)) || (rc = check_opts(grid, opts))) return rc;
   if (tracks->n_particles == 0) return SR_OK;
-  const Plan pl = make_plan(*grid, *opts, tracks->n_particles, tracks->n_snaps, tracks->n_points);
+  const Plan pl = make_plan(*grid, *opts, tracks->n_particles, tracks->n_snaps, tracks->n_points, mean_steps(*tracks));
   *bytes = scratch_bytes(pl, outputs_for(grid->mode, opts->comp),
                          (int64_t)grid->n_omega * grid->n_theta * grid->n_phi, tracks->n_snaps) +
            pre_bytes(grid->mode, tracks->n_points) + order_bytes(pl, *grid, *opts, tracks->n_points);
@@ -1463,7 +1524,7 @@ int sr_spectrum_batch(const sr_tracks *t, const sr_grid *g, const sr_opts *o, do
   kp.dt = t->dt;
   kp.n_points = t->n_points;
   fill_grid(kp, *g, *o, n_out, outs);
-  const Plan pl = make_plan(*g, *o, t->n_particles, t->n_snaps, t->n_points);
+  const Plan pl = make_plan(*g, *o, t->n_particles, t->n_snaps, t->n_points, mean_steps(*t));
   slice_particles(kp, pl.slices, t->n_particles, t->offsets_host);
   return run(kp, pl, *g, *o, workspace, workspace_bytes, (hipStream_t)stream, true,
              order_bytes(pl, *g, *o, t->n_points));
@@ -1474,7 +1535,7 @@ int sr_plan(const sr_tracks *t, const sr_grid *g, const sr_opts *o, sr_plan_info
   if (!info) return fail(SR_ERR_INVALID, "info is NULL");
   memset(info, 0, sizeof(*info));
   if ((rc = check_tracks(t)) || (rc = check_grid(g)) || (rc = check_opts(g, o))) return rc;
-  const Plan pl = make_plan(*g, *o, std::max<int64_t>(t->n_particles, 1), t->n_snaps, t->n_points);
+  const Plan pl = make_plan(*g, *o, std::max<int64_t>(t->n_particles, 1), t->n_snaps, t->n_points, mean_steps(*t));
   info->sweep = pl.sweep == SWEEP_REC ? SR_SWEEP_RECURRENCE : SR_SWEEP_DIRECT;
   info->omega_per_lane = pl.M;
   info->waves_per_block = pl.waves;
@@ -1586,7 +1647,7 @@ int sr_spectrum_batch_noalloc(const sr_tracks *t, const sr_grid *g, const sr_opt
   kp.dt = t->dt;
   kp.n_points = t->n_points;
   fill_grid(kp, *g, *o, n_out, outs);
-  Plan pl = make_plan(*g, *o, t->n_particles, t->n_snaps, t->n_points);
+  Plan pl = make_plan(*g, *o, t->n_particles, t->n_snaps, t->n_points, mean_steps(*t));
   // the same plan as sr_spectrum_batch; a tuned slice count is halved until
   // the slices' partial spectra and the tile order fit the scratch array
   auto need = [&](const Plan &p) {

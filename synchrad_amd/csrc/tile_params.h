@@ -48,6 +48,9 @@ struct KParams {
   uint32_t n_dir;
   UDiv div_chunks, div_dir, div_theta;   // by n_chunks, n_dir, n_theta (tiles < 2^31)
   int32_t slices;
+  // tile kernel, FP64: the block's groups of threads that share a tile, each
+  // sweeping a contiguous part of every track
+  int32_t parts;
   int64_t n_tiles;
   int64_t slice_lo[kMaxSlices + 1];
   // launch order of the tiles (heaviest first), or nullptr: index order
