@@ -24,13 +24,14 @@
 // applies the m, a -> b -> u chain: no atomics, and the result does not depend
 // on scheduling.
 //
-// Split precision, ascending non-negative linear grid: a step keeps exactly the
-// omegas below its threshold |omega|/2pi < 1/(2 |tau_s - tau_{s-1}|) (the
-// forward's test), a prefix of the table found by binary search; exp(i omega
-// tau) walks the prefix by rotation with exp(i domega tau), restarted from an
-// FP64 phase every 32 omegas.  'total' keeps the coefficients on e_theta,
-// e_phi (F is perpendicular to n).  FP64 keeps the reference's exact per-pair
-// test and an FP64 sin/cos per pair.
+// Split precision on a linear grid, tracks of some hundred steps and more: the
+// transpose sweep as matrix products (adjoint_factored.h).  Shorter tracks, ascending
+// non-negative linear grid: a step keeps exactly the omegas below its threshold
+// |omega|/2pi < 1/(2 |tau_s - tau_{s-1}|) (the forward's test), a prefix of the table
+// found by binary search; exp(i omega tau) walks the prefix by rotation with exp(i
+// domega tau), restarted from an FP64 phase every 32 omegas.  'total' keeps the
+// coefficients on e_theta, e_phi (F is perpendicular to n).  FP64 keeps the
+// reference's exact per-pair test and an FP64 sin/cos per pair.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -80,11 +81,23 @@ struct AParams {
   // decomposition and workspace
   int32_t n_groups;
   int32_t dir_batch;   // directions whose coefficient tables share the block's LDS
+  // factored sweep: blocks that share a particle's steps, groups of 32 omegas per
+  // table, omega tiles, the direction range whose tables are in `tab`, and the direction
+  // groups of the weights' sums
+  int32_t n_ranges, tile_groups, n_wtiles, n_wgroups;
+  uint32_t dir_lo, dir_n;
+  char *tab;
   double *slab;    // [n_groups][kSlabWords][n_points]
-  double *slab_w;  // [n_groups][n_particles]
+  double *slab_w;  // [n_wgroups][n_particles]
   // outputs (+=)
   double *gx, *gy, *gz, *gux, *guy, *guz, *gw;
 };
+
+}  // namespace
+
+#include "adjoint_factored.h"
+
+namespace {
 
 // frequencies per iteration of the transpose sweep's direct omega loop
 #ifndef SR_ADJ_UNROLL
@@ -411,7 +424,7 @@ __global__ void k_adjoint_reduce_w(const AParams p) {
   const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (ip >= p.n_particles) return;
   double s = 0.0;
-  for (int q = 0; q < p.n_groups; q++) s += p.slab_w[(int64_t)q * p.n_particles + ip];
+  for (int q = 0; q < p.n_wgroups; q++) s += p.slab_w[(int64_t)q * p.n_particles + ip];
   p.gw[ip] += s;
 }
 
@@ -457,15 +470,24 @@ __global__ void k_fields_spectrum(const int64_t *offsets, const double *weight, 
 }
 
 struct APlan {
+  bool factored;   // split precision on a linear grid (adjoint_factored.h)
   int threads;
   int groups;
   int64_t chunk;   // particles whose fields share the workspace at once
   int dir_batch;   // directions per LDS batch
+  int ranges;      // factored: blocks that share a particle's steps
+  int tile_groups; // factored: groups of 32 omegas per table
+  int wgroups;     // direction groups of the weights' sums
+  int64_t tab_dirs;   // factored: directions whose tables share the workspace at once
+  size_t tab_bytes;   // and their size
+  size_t tab_lds;
   size_t lds;      // dynamic LDS of the sweep kernel
 };
 
 // LDS for the coefficient tables of one direction batch
 constexpr size_t kAdjTableBudget = 32768;
+// the factored sweep's tables of a launch: as large as the last-level cache
+constexpr double kAdjTablesBytes = 268435456.0;
 
 // fields of one chunk of particles: 6 doubles per (particle, point), ~2 GiB at most
 constexpr double kFieldBudget = 2147483648.0;
@@ -473,20 +495,63 @@ constexpr double kFieldBudget = 2147483648.0;
 // all_fields: the caller holds every particle's fields (one chunk)
 APlan adjoint_plan(const sr_tracks &t, const sr_grid &g, const sr_opts &o, bool all_fields) {
   APlan pl;
-  // threads = steps of the transpose sweep
-  const int waves = o.waves_per_block > 0 ? o.waves_per_block : 4;
+  const bool split = o.precision == SR_PREC_SPLIT;
+  pl.ranges = 1;
+  pl.tile_groups = 0;
+  // threads = steps of the transpose sweep; factored: four waves, as far as the
+  // tracks fill them
+  const int64_t steps = t.n_particles > 0 ? t.n_points / t.n_particles : 0;
+  // matrix products from the track length on at which a direction's table is paid for:
+  // betatron beams, forward and adjoint, rotation loop -> matrix products, 'total' 100 x
+  // 500 steps on 64 x 16 x 16 1.06 -> 0.97 ms, 300 x 150 on 40 x 10 x 10 0.68 -> 0.72;
+  // 'cartesian', three words in two half-filled sets, 64 x 4000 on 128 x 32 x 32 21.6 ->
+  // 17.2, 100 x 500 on 64 x 16 x 16 1.12 -> 1.20, 8 x 1000 on 24 x 16 x 16 0.54 -> 0.57
+  const bool total = o.comp == SR_COMP_TOTAL;
+  pl.factored = split && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) && g.n_omega >= (total ? 24u : 64u);
+  int waves = 4;
+  if (pl.factored) {
+    waves = kAdjMaxT / kWave;
+    while (waves > 1 && steps <= kWave * waves / 2) waves /= 2;
+  }
+  if (o.waves_per_block > 0) waves = o.waves_per_block;
   pl.threads = kWave * waves;
   const int64_t n_dir = (int64_t)g.n_theta * g.n_phi;
   const int64_t n_grid = n_dir * g.n_omega;
   pl.chunk = all_fields ? std::max<int64_t>(1, t.n_particles)
                         : std::max<int64_t>(1, std::min<int64_t>(t.n_particles,
                                                                  (int64_t)(kFieldBudget / (48.0 * n_grid))));
-  int64_t groups = o.slices > 0 ? o.slices : std::max<int64_t>(1, (4096 + pl.chunk - 1) / pl.chunk);
+  // blocks of a particle: direction groups and (factored) runs of steps, until there are
+  // 4096 blocks, or 16K waves (factored)
+  int64_t want = 4096;
+  if (pl.factored) {
+    pl.ranges = (int)std::min<int64_t>(std::max<int64_t>(1, (steps + pl.threads - 1) / pl.threads), 1 << 12);
+    want = 16384 / waves;
+  }
+  const int64_t have = pl.chunk * pl.ranges;
+  int64_t groups = o.slices > 0 ? o.slices : std::max<int64_t>(1, (want + have - 1) / have);
   pl.groups = (int)std::min<int64_t>(std::min<int64_t>(groups, n_dir), 1 << 16);
-  const bool split = o.precision == SR_PREC_SPLIT;
+  const int64_t dirs_per_group = (n_dir + pl.groups - 1) / pl.groups;
+  pl.wgroups = pl.groups;
+  pl.tab_dirs = n_dir;
+  pl.tab_bytes = 0;
+  pl.tab_lds = 0;
+  if (pl.factored) {
+    const int max_groups = total ? adj_tile_groups<true>() : adj_tile_groups<false>();
+    pl.tile_groups = (int)std::min<int64_t>(max_groups, ((int64_t)g.n_omega + 2 * kGroup - 1) / (2 * kGroup) * 2);
+    const int64_t tile = (int64_t)pl.tile_groups * kGroup;
+    const int64_t wtiles = ((int64_t)g.n_omega + tile - 1) / tile;
+    const size_t rec = total ? AdjRecord<true>{pl.tile_groups}.bytes() : AdjRecord<false>{pl.tile_groups}.bytes();
+    pl.tab_dirs = std::max<int64_t>(1, std::min<int64_t>(n_dir, (int64_t)(kAdjTablesBytes / (double)(rec * wtiles * pl.chunk))));
+    pl.groups = (int)std::min<int64_t>(pl.groups, pl.tab_dirs);
+    pl.tab_bytes = rec * (size_t)wtiles * (size_t)pl.chunk * (size_t)pl.tab_dirs;
+    pl.wgroups = (int)std::min<int64_t>(std::max<int64_t>(1, (8192 + pl.chunk - 1) / pl.chunk), pl.tab_dirs);
+    pl.tab_lds = kTabWaves * rec;
+    pl.dir_batch = 1;
+    pl.lds = adj_lds_bytes(waves, pl.tile_groups);
+    return pl;
+  }
   const size_t per_dir = (size_t)((o.comp == SR_COMP_TOTAL) ? 4 : 6) * std::min<uint32_t>(g.n_omega, kAdjOmegaTile) *
                          (split ? sizeof(float) : sizeof(double));
-  const int64_t dirs_per_group = (n_dir + pl.groups - 1) / pl.groups;
   pl.dir_batch = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)(kAdjTableBudget / per_dir), 16,
                                                               dirs_per_group}));
   pl.lds = per_dir * pl.dir_batch;
@@ -520,15 +585,15 @@ int adjoint_check(const sr_tracks *t, const sr_grid *g, const sr_opts *o) {
 }
 
 size_t adjoint_slab_words(const sr_tracks &t, const APlan &pl) {
-  return (size_t)pl.groups * kSlabWords * (size_t)t.n_points + (size_t)pl.groups * (size_t)t.n_particles;
+  return (size_t)pl.groups * kSlabWords * (size_t)t.n_points + (size_t)pl.wgroups * (size_t)t.n_particles;
 }
 
-// workspace: slabs, the fields of one chunk of particles (unless the caller
+// workspace: the factored sweep's tables, slabs, the fields of one chunk of particles (unless the caller
 // passes them), the step data, and (with own fields) the fields launches' tile
 // order
 size_t adjoint_ws(const sr_tracks &t, const sr_grid &g, const APlan &pl, bool own_fields, int32_t precision) {
   const size_t n_grid = (size_t)g.n_omega * g.n_theta * g.n_phi;
-  return (adjoint_slab_words(t, pl) + (own_fields ? 6 * (size_t)pl.chunk * n_grid : 0) +
+  return pl.tab_bytes + (adjoint_slab_words(t, pl) + (own_fields ? 6 * (size_t)pl.chunk * n_grid : 0) +
           6 * (size_t)t.n_points) * sizeof(double) +
          (own_fields ? fields_order_space(t, g, precision, pl.chunk) : 0);
 }
@@ -571,10 +636,15 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
   for (int c = 0; c < 3; c++) p.dS[c] = dS[c < n_in ? c : 0];
   p.n_groups = pl.groups;
   p.dir_batch = pl.dir_batch;
-  p.slab = (double *)workspace;
+  p.n_ranges = pl.ranges;
+  p.tile_groups = pl.tile_groups;
+  p.n_wgroups = pl.wgroups;
+  p.n_wtiles = pl.factored ? (int)((p.n_omega + pl.tile_groups * kGroup - 1) / (pl.tile_groups * kGroup)) : 1;
+  p.tab = (char *)workspace;
+  p.slab = (double *)(p.tab + pl.tab_bytes);
   p.slab_w = p.slab + (size_t)pl.groups * kSlabWords * (size_t)t->n_points;
   p.gx = gx; p.gy = gy; p.gz = gz; p.gux = gux; p.guy = guy; p.guz = guz; p.gw = gw;
-  double *fields = (double *)workspace + adjoint_slab_words(*t, pl);
+  double *fields = p.slab + adjoint_slab_words(*t, pl);
   double *pre = own ? fields + 6 * (size_t)pl.chunk * (size_t)p.n_grid : fields;
   void *order_ws = own ? (void *)(pre + 6 * (size_t)t->n_points) : nullptr;
   const size_t order_space = own ? fields_order_space(*t, *g, o->precision, pl.chunk) : 0;
@@ -582,7 +652,8 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
   p.pre = pre;
   hipStream_t st = (hipStream_t)stream;
   const int64_t n_clear = (int64_t)adjoint_slab_words(*t, pl);
-  hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)((n_clear + 255) / 256)), dim3(256), 0, st, p.slab, n_clear);
+  if (!pl.factored)   // (the factored sweep's tables clear them)
+    hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)((n_clear + 255) / 256)), dim3(256), 0, st, p.slab, n_clear);
   if ((rc = step_prep(*t, SR_MODE_FAR, pre, st))) return rc;
   for (int64_t pb = 0; pb < t->n_particles; pb += pl.chunk) {
     const int64_t pe = std::min<int64_t>(t->n_particles, pb + pl.chunk);
@@ -593,8 +664,21 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
     }
     p.chunk_base = pb;
     p.chunk_n = pe - pb;
-    const int64_t blocks = p.chunk_n * (int64_t)pl.groups;
-    if (o->precision == SR_PREC_F64 && o->comp == SR_COMP_TOTAL)
+    const int64_t blocks = p.chunk_n * (int64_t)pl.groups * pl.ranges;
+    if (pl.factored) {
+      const int64_t tab_blocks = (p.chunk_n * pl.wgroups + kTabWaves - 1) / kTabWaves;
+      for (int64_t db = 0; db < (int64_t)p.n_dir; db += pl.tab_dirs) {
+        p.dir_lo = (uint32_t)db;
+        p.dir_n = (uint32_t)std::min<int64_t>(pl.tab_dirs, (int64_t)p.n_dir - db);
+        if (o->comp == SR_COMP_TOTAL) {
+          hipLaunchKernelGGL((k_adjoint_tables<true>), dim3((unsigned)tab_blocks), dim3(kTabWaves * kWave), pl.tab_lds, st, p);
+          hipLaunchKernelGGL((k_adjoint_factored<true>), dim3((unsigned)blocks), dim3(pl.threads), pl.lds, st, p);
+        } else {
+          hipLaunchKernelGGL((k_adjoint_tables<false>), dim3((unsigned)tab_blocks), dim3(kTabWaves * kWave), pl.tab_lds, st, p);
+          hipLaunchKernelGGL((k_adjoint_factored<false>), dim3((unsigned)blocks), dim3(pl.threads), pl.lds, st, p);
+        }
+      }
+    } else if (o->precision == SR_PREC_F64 && o->comp == SR_COMP_TOTAL)
       hipLaunchKernelGGL((k_adjoint<SR_PREC_F64, true>), dim3((unsigned)blocks), dim3(pl.threads), pl.lds, st, p);
     else if (o->precision == SR_PREC_F64)
       hipLaunchKernelGGL((k_adjoint<SR_PREC_F64, false>), dim3((unsigned)blocks), dim3(pl.threads), pl.lds, st, p);
