@@ -20,8 +20,10 @@
 // threshold.  Tiles that no step of the wave keeps a whole group of are skipped, groups
 // that a step does not keep whole are left out of its combination, and a group that steps
 // cut (on betatron tracks four waves in five have one, rarely two) is a second product
-// with the basis masked step by step.  There the two sides +-beta_b of the group are
-// needed apart; the lower side's table is formed from the group's own.
+// with the basis masked step by step: of the table's two sides +-beta_b apart, eight rows
+// each, only the side that the step cuts, added to nothing or taken off the whole group.
+// (Both sides in a product of their own, 24 matrix instructions a group instead of 12: the
+// backward of 256 electrons x 4000 steps on 128 x 32 x 32 33.3 ms against 30.0.)
 //
 // Work split: a first kernel forms each (particle, direction)'s coefficient table in the
 // matrix operand's order, a wave a table; then a block owns (particle, direction group,
@@ -36,7 +38,7 @@
 //
 // Bound: vector instructions (FP64 step geometry and gradient chain about a third, the
 // basis' word pairs about a third) with the matrix products beneath.  64 betatron
-// electrons x 4000 steps on 128 x 32 x 32: 6.0 ms and 0.17 ms for the tables, against
+// electrons x 4000 steps on 128 x 32 x 32: 5.9 ms and 0.17 ms for the tables, against
 // 8.6 ms of the rotation loop; summing the cut groups frequency by frequency in FP32
 // instead of the masked product 7.5 ms.
 #pragma once
@@ -82,18 +84,14 @@ struct AdjRecord {
 };
 // LDS of a sweep block: the waves' own, the frequencies, the group bounds
 constexpr size_t adj_lds_bytes(int waves, int ng) {
-  return (size_t)waves * kAdjWaveBytes + (size_t)ng * (kGroup + 3) * 8;
+  return (size_t)waves * kAdjWaveBytes + (size_t)ng * (kGroup + 3) * 8 + 16;
 }
-// a bit per value, two of them, as a mask of two packed halves
-__device__ __forceinline__ uint32_t halves(uint32_t bits) {
-  const uint32_t lo = (uint32_t)((int32_t)(bits << 31) >> 31), hi = (uint32_t)((int32_t)(bits << 30) >> 31);
-  return (lo & 0xffffu) | (hi & 0xffff0000u);
-}
-// The part of a group's table that belongs to the offsets -beta_b.  A lane holds a row's
-// 4 cos and 4 sin columns, its neighbour (lane ^ 1) the group's other row; with the row of
+// A group's table as two, of the offsets -beta_b and +beta_b apart.  A lane holds a row's 4
+// cos and 4 sin columns, its neighbour (lane ^ 1) the group's other row; with the row of
 // cos(alpha tau) (a+ + a-, b+ - b-) and that of sin(alpha tau) (b+ + b-, a- - a+), the
-// lower parts are (a-, -b-) and (b-, a-)
-__device__ __forceinline__ void lower_side(uint4v th, uint4v tl, float one, uint4v *lh, uint4v *ll) {
+// lower parts are (a-, -b-) and (b-, a-), the upper ones the rest.  Lanes with bit 1 clear
+// form the lower part of their row, the others the upper
+__device__ __forceinline__ void two_sides(uint4v th, uint4v tl, float one, uint4v *oh, uint4v *ol) {
   float v[8];
 #pragma unroll
   for (int k = 0; k < 4; k++) {
@@ -101,7 +99,8 @@ __device__ __forceinline__ void lower_side(uint4v th, uint4v tl, float one, uint
     v[2 * k] = ((float)h.x + (float)l.x) * 0.5f;
     v[2 * k + 1] = ((float)h.y + (float)l.y) * 0.5f;
   }
-  const float sg = (threadIdx.x & 1) ? -1.f : 1.f;
+  const int ln = (int)threadIdx.x;
+  const float sg = ((ln ^ (ln >> 1)) & 1) ? -1.f : 1.f;
   float u[8];
 #pragma unroll
   for (int k = 0; k < 8; k++) {
@@ -112,8 +111,8 @@ __device__ __forceinline__ void lower_side(uint4v th, uint4v tl, float one, uint
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     const uint2 w = split_values(u[2 * k], u[2 * k + 1], one);
-    (*lh)[k] = w.x;
-    (*ll)[k] = w.y;
+    (*oh)[k] = w.x;
+    (*ol)[k] = w.y;
   }
 }
 // waves of a table block
@@ -275,6 +274,8 @@ k_adjoint_factored(const AParams p) {
   double *const s_alpha = (double *)carve((size_t)ng * 8);                            // group centres / 2pi
   double *const s_lo = (double *)carve((size_t)ng * 8);                               // bounds of |omega| / 2pi
   double *const s_hi = (double *)carve((size_t)ng * 8);
+  uint32_t *const s_cross = (uint32_t *)carve(16);   // groups on both sides of zero, groups of ascending |omega|
+  auto s_up = [&](int g) { return ((s_cross[1] >> g) & 1u) != 0; };
   char *const s_own = ptr + wv * kAdjWaveBytes;
   float2 *const s_fac = (float2 *)s_own;        // [7][kAdjRow]: e^{i (4 k1 + 1/2) d}, e^{i k0 d}
   float4 *const s_al = (float4 *)s_own;         // then, twice [64]: cos, sin of two group centres
@@ -300,25 +301,16 @@ k_adjoint_factored(const AParams p) {
   double *slab = p.slab + (int64_t)q_dir * kSlabWords * p.n_points;
 
   int n_om = 0;
-  // which of group g's frequencies a step of threshold thr keeps, bit j the j-th.  On a
-  // linear grid their count in ascending |omega| is known to one, and the threshold's own
-  // comparison settles it
-  auto kept_of = [&](int g, bool mine, double thr) -> uint32_t {
+  // how many of group g's frequencies a step of threshold thr keeps, those of smallest
+  // |omega|; the group's |omega| ascend (up) or descend.  On a linear grid the count is
+  // known to one, and the threshold's own comparison settles it
+  auto kept_of = [&](int g, bool up, double thr) -> int {
     const double *w = s_om + g * kGroup;
     const int cnt = min(kGroup, n_om - g * kGroup);
-    const double w0 = w[0], w1 = w[cnt - 1];
-    uint32_t kept = 0;
-    if ((w0 < 0.0) == (w1 < 0.0)) {
-      const bool up = fabs(w1) >= fabs(w0);
-      int r = min((int)fmin(fmax((thr - fmin(fabs(w0), fabs(w1))) * step_inv, 0.0), 31.0) + 1, cnt - 1);
-      if (!mine) r = 0;
-      const double in = fabs(w[up ? max(r - 1, 0) : cnt - max(r, 1)]), out = fabs(w[up ? r : cnt - 1 - r]);
-      r += (out < thr && r < cnt - 1) ? 1 : (!(in < thr) && r > 0) ? -1 : 0;
-      kept = ((1u << r) - 1u) << (up ? 0 : cnt - r);
-    } else {
-      for (int j = 0; j < cnt; j++) kept |= (uint32_t)(fabs(w[j]) < thr) << j;
-    }
-    return mine ? kept : 0u;
+    int r = min((int)fmin(fmax((thr - s_lo[g]) * step_inv, 0.0), 31.0) + 1, cnt - 1);
+    const double in = fabs(w[up ? max(r - 1, 0) : cnt - max(r, 1)]), out = fabs(w[up ? r : cnt - 1 - r]);
+    // (past the grid's end a descending group's frequencies count as kept: zeros)
+    return r + ((out < thr && r < cnt - 1) ? 1 : (!(in < thr) && r > 0) ? -1 : 0) + (up ? 0 : kGroup - cnt);
   };
 
   for (int64_t base = (int64_t)rg * T; base < n_use; base += (int64_t)n_ranges * T) {
@@ -350,6 +342,8 @@ k_adjoint_factored(const AParams p) {
     const int w0 = wt * ng * kGroup;
     n_om = min(ng * kGroup, (int)p.n_omega - w0);
     __syncthreads();   // the previous omega tile's bounds are read
+    if (tid < 2) s_cross[tid] = 0;
+    __syncthreads();
     for (int i = tid; i < ng * kGroup; i += T) s_om[i] = i < n_om ? p.omega[w0 + i] * kInv2Pi : 0.0;
     for (int i = tid; i < ng; i += T) {
       const int first = i * kGroup, last = min(first + kGroup, n_om) - 1;
@@ -358,7 +352,12 @@ k_adjoint_factored(const AParams p) {
         const double wa = p.omega[w0 + first] * kInv2Pi, wb = p.omega[w0 + last] * kInv2Pi;
         al = fma(15.5, p.domega_rev, wa);
         hi = fmax(fabs(wa), fabs(wb));
-        lo = (wa < 0.0) == (wb < 0.0) ? fmin(fabs(wa), fabs(wb)) : 0.0;
+        lo = fmin(fabs(wa), fabs(wb));
+        if (fabs(wb) >= fabs(wa)) atomicOr(&s_cross[1], 1u << i);
+        if ((wa < 0.0) != (wb < 0.0)) {
+          lo = 0.0;
+          atomicOr(&s_cross[0], 1u << i);
+        }
       }
       s_alpha[i] = al; s_lo[i] = lo; s_hi[i] = hi;
     }
@@ -416,12 +415,29 @@ k_adjoint_factored(const AParams p) {
         const bool cuts = __ballot(!all_kept) != 0;
         double thr = 0.0;
         uint32_t whole = 0, part = 0;
+        uint32_t slow = 0;           // cut groups that the masked product does not take
+        int cut_at = 0, cut_r = 0;   // the lane's cut group and its kept count
         if (cuts) {
           thr = 0.5 / dtau;
           for (int g = 0; g < ng; g++) {
             const uint32_t w = s_hi[g] < thr, l = s_lo[g] < thr;
             whole |= w << g;
             part |= (l & ~w) << g;
+          }
+          // a step that keeps more than half of the group it cuts takes it whole, less the
+          // offsets of one side that it drops; else it takes the kept offsets of one side.
+          // Groups on both sides of zero and coefficients that are not finite go apart
+          if (part != 0) {
+            const uint32_t odd = *(const uint32_t *)(rec_at + rec.flag_at()) | *s_cross;
+            slow = part & odd;
+            part &= ~odd;
+            slow |= part & (part - (part != 0));   // (a grid across zero can be cut on both sides)
+            if (part != 0) {
+              cut_at = __builtin_ctz(part);
+              cut_r = kept_of(cut_at, s_up(cut_at), thr);
+              part = 1u << cut_at;
+              if (cut_r > 16) whole |= part;
+            }
           }
           s_msk[lane] = whole;
         }
@@ -536,61 +552,52 @@ k_adjoint_factored(const AParams p) {
           }
           t = next;
         }
-        // the groups that steps of the wave cut, mostly one: table times the basis of the
-        // offsets kept on the upper side, plus the table of the lower side alone times the
-        // basis of the offsets kept there only (minus where on the upper side only)
-        uint32_t slow = 0;           // this lane's cut groups with coefficients that are not finite
+        // the groups that steps of the wave cut, mostly one: the table's two sides, eight rows
+        // each, times the basis masked to the offsets from |16 - kept| on -- the side kept if
+        // that is less than half of the group, the side dropped, to be subtracted, if more
         if (cuts) {
-          uint32_t odd = 0;
           for (int g = 0; g < ng; g++) {
-            const bool mine = (part >> g) & 1u;
+            const bool mine = part != 0 && cut_at == g;
             if (__ballot(mine) == 0) continue;
-            if (odd == 0) odd = 0x80000000u | (uint32_t)uni(*(const int *)(rec_at + rec.flag_at()));
-            if ((odd >> g) & 1u) {
-              slow |= mine ? 1u << g : 0u;
-              continue;
-            }
-            const uint32_t kept = kept_of(g, mine, thr);
+            const bool up = s_up(g);
             float2 ph;
             sincos_rev(s_alpha[g] * tau, &ph.y, &ph.x);
+            const bool more = cut_r > 16;
+            const float low = mine && (more != up) ? 1.f : 0.f, high = mine && (more == up) ? 1.f : 0.f;
+            const float sgn = more ? -1.f : 1.f;
+            const uint32_t from = mine ? (uint32_t)(more ? cut_r - 16 : 16 - cut_r) : 16u;
             sr::wave_sync();
-            s_msk[lane] = kept;
-            s_fac[lane] = ph;
+            s_msk[lane] = from | (from << 16);
+            s_al[lane] = make_float4(sgn * low * ph.x, sgn * low * ph.y, sgn * high * ph.x, sgn * high * ph.y);
             sr::wave_sync();
 #pragma unroll
             for (int set = 0; set < NSET; set++) {
-              const uint4v *tb = tab + ((g >> 1) * NSET + set) * 2 * kWave;
-              const uint4v gh = tb[0], gl = tb[kWave];
-              uint4v lh, ll;
-              lower_side(gh, gl, one, &lh, &ll);
+              const uint4v *tb = (const uint4v *)rec_at + ((g >> 1) * NSET + set) * 2 * kWave + ((lane & ~2) | (2 * (g & 1)));
+              uint4v gh, gl;
+              two_sides(tb[0], tb[kWave], one, &gh, &gl);
               const float sc = scl[(g * NSET + set) * 4];
 #pragma unroll
               for (int blk = 0; blk < 4; blk++) {
-                const uint32_t kb = s_msk[16 * blk + col];
-                const float2 al = s_fac[16 * blk + col];
-                const uint32_t up = kb >> (16 + 4 * quad), down = __builtin_bitreverse32(kb) >> (16 + 4 * quad);
-                uint4v ph4, pl4, mh4, ml4;
+                const short2v fr = __builtin_bit_cast(short2v, s_msk[16 * blk + col]);
+                const float4 al = s_al[16 * blk + col];
+                uint4v mh, ml;
 #pragma unroll
                 for (int k = 0; k < 2; k++) {
-                  const uint32_t mp = halves(up >> (2 * k)), mm = halves(down >> (2 * k));
-                  const uint32_t only = mp ^ mm, sg = mp & ~mm & 0x80008000u;
+                  // offsets 4 quad + 2 k, + 1: all ones where from <= offset
+                  const short b0 = (short)(4 * quad + 2 * k + 1);
+                  const short2v off = {b0, (short)(b0 + 1)};
+                  const uint32_t mm = __builtin_bit_cast(uint32_t, (short2v)((fr - off) >> 15));
 #pragma unroll
                   for (int h = 0; h < 4; h += 2) {
-                    ph4[h + k] = bh[blk][h + k] & mp;
-                    pl4[h + k] = bl[blk][h + k] & mp;
-                    mh4[h + k] = (bh[blk][h + k] ^ sg) & only;
-                    ml4[h + k] = (bl[blk][h + k] ^ sg) & only;
+                    mh[h + k] = bh[blk][h + k] & mm;
+                    ml[h + k] = bl[blk][h + k] & mm;
                   }
                 }
-                float4v U = mfma16(gl, ph4, (float4v)(0.f));
-                U = mfma16(ll, mh4, U);
-                U = mfma16(gh, pl4, U);
-                U = mfma16(lh, ml4, U);
-                U = mfma16(gh, ph4, U);
-                U = mfma16(lh, mh4, U);
-                const float x = (g & 1) ? U[2] : U[0], y = (g & 1) ? U[3] : U[1];
-                const float u = __builtin_fmaf(al.x, x, al.y * y);
-                out[set][blk] = kb != 0 ? __builtin_fmaf(sc, u, out[set][blk]) : out[set][blk];
+                float4v U = mfma16(gl, mh, (float4v)(0.f));
+                U = mfma16(gh, ml, U);
+                U = mfma16(gh, mh, U);
+                const float u = __builtin_fmaf(al.x, U[0], al.y * U[1]) + __builtin_fmaf(al.z, U[2], al.w * U[3]);
+                out[set][blk] = __builtin_fmaf(sc, u, out[set][blk]);
               }
             }
           }
@@ -608,8 +615,7 @@ k_adjoint_factored(const AParams p) {
           P[c] = s_out[c * kWave + lane];
           R[c] = s_out[(TWO ? NCW + c : 4 + c) * kWave + lane];
         }
-        // cut groups with coefficients that are not finite: only the frequencies that are
-        // kept may be touched
+        // the cut groups left: only the frequencies that are kept may be touched
         while (slow != 0) {
           const int g = __builtin_ctz(slow);
           slow &= slow - 1;

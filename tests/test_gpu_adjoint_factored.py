@@ -91,3 +91,9 @@ def test_coefficients_that_are_not_finite_stay_with_the_steps_that_keep_them():
     a, b = (_grads(wl.batch, grid, [G], "total", prec) for prec in ("float", "double"))
     for c in range(3):
         assert torch.equal(torch.isfinite(a[c]), torch.isfinite(b[c]))
+
+
+def test_tables_of_several_launches():
+    """More tables than fit at once: 90 electrons, 32 x 32 directions, 128 frequencies."""
+    wl = workloads.config2(n_particles=90, n_steps=390, grid=(128, 32, 32))
+    _check(wl, wl.axes)
