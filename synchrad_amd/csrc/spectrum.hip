@@ -1006,11 +1006,15 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   // AUTO: the factored tiles for split spectra on linear grids, except far-field
   // grids of at most one 64-omega wave: there the direct sweep's sine per omega
   // costs no more than forming the factors (32 betatron electrons on 64 x 32 x 32:
-  // 3.38 ms against 3.62; on 72 omegas 6.8 against 3.6)
+  // 3.38 ms against 3.62; on 72 omegas 6.8 against 3.6).  Long tracks on too few
+  // directions to fill the GPU take them there too: the direct sweep has no more waves
+  // than tiles, a factored tile's steps are shared by four (one electron x 6000 steps on
+  // 24 x 20 x 4 495 us against 86)
+  const int64_t spread = n_dir * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices);
   pl.sweep = SWEEP_DIRECT;
   if (o.precision == SR_PREC_SPLIT && g.omega_step != 0.0 &&
       (o.sweep == SR_SWEEP_RECURRENCE ||
-       (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave))))
+       (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave || (mean_steps >= 1008 && spread < 2048)))))
     pl.sweep = SWEEP_REC;
   // FP64: groups of threads that may share a tile's steps: blocks of at most
   // kMaxParts waves, two staged tiles of steps for each
@@ -1041,10 +1045,15 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
     // (betatron beam, 24 x 8000 steps on 512 x 32 x 32: 8.1 ms against 9.1; the
     // near-field screen with 4 groups the other way, 6.9 against 7.6), and more
     // where the tiles and particle slices leave the GPU short of waves (one
-    // undulator electron on 256 x 32 x 32: 71 us with two, 94 with one)
-    pl.waves = pl.groups == 16 ? 2 : 1;
-    while (pl.waves < 4 &&
-           chunks * n_dir * pl.waves * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices) < 2048)
+    // undulator electron on 256 x 32 x 32: 71 us with two, 94 with one), as long as a
+    // wave has four stages' steps of each track: each fills queues of its own (30 x 200
+    // steps on 600 x 40 x 20, three words: 0.71 ms with one, 1.08 with two; 100 x 400 on
+    // 512 x 16 x 16 0.68 against 0.82); one stage each where even the tiles of two waves
+    // leave half of the CUs without one
+    auto shared = [&](int w, int stages) { return mean_steps >= (int64_t)w * stages * (kWave - 1); };
+    pl.waves = pl.groups == 16 && shared(2, 4) ? 2 : 1;
+    while (pl.waves < 4 && ((shared(2 * pl.waves, 4) && chunks * pl.waves * spread < 2048) ||
+                            (shared(2 * pl.waves, 1) && chunks * pl.waves * spread < 512)))
       pl.waves *= 2;
     if (o.waves_per_block > 0) pl.waves = o.waves_per_block;
   } else {
