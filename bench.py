@@ -45,6 +45,7 @@ METRIC = "G spectral-pt×step evals/s: split-FP32 vs FP64 @≤1e-4 relL2; % vect
 FLOP_PER_EVAL = {"far": 49.0, "near": 54.0}
 PEAK_FP32_TFLOPS = 157.3
 PEAK_FP64_TFLOPS = 78.6
+PEAK_FP16_MATRIX_TFLOPS = 2500.0   # dense
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "tile_kernel_betatron_traffic.md")
 COUNTERS_FILE = os.path.join(REPO, "profiles", "tile_kernel_betatron_counters.md")
 ADJOINT_COUNTERS_FILE = os.path.join(REPO, "profiles", "adjoint_betatron_counters.md")
@@ -209,7 +210,9 @@ def executed_roofline(kind, kernel_ms, path=COUNTERS_FILE):
     apart), divided by the launch time measured now.  ``frac`` is the share of
     the launch the vector ALUs would need at their peaks for that work, FP32
     at 157.3 TFLOP/s plus FP64 at 78.6 -- achieved is stated in FP32-equivalent
-    TFLOP/s (an FP64 flop counted as two, the ratio of the peaks)."""
+    TFLOP/s (an FP64 flop counted as two, the ratio of the peaks).  The fp16
+    matrix work beneath it (512 flops per counted MOP) is stated beside it
+    against the dense fp16 peak, and is not part of ``frac``."""
     c = counters_from_profile(kind, path)
     if not c:
         return None
@@ -224,6 +227,10 @@ def executed_roofline(kind, kernel_ms, path=COUNTERS_FILE):
            "achieved_fp32_equiv": round(a32 + 2 * a64, 3),
            "frac": round(a32 / PEAK_FP32_TFLOPS + a64 / PEAK_FP64_TFLOPS, 4),
            "flop_fp32_per_launch": f32, "flop_fp64_per_launch": f64}
+    if "SQ_INSTS_VALU_MFMA_MOPS_F16" in c:
+        a16 = 512.0 * c["SQ_INSTS_VALU_MFMA_MOPS_F16"] / t / 1e12
+        out["matrix_fp16_tflops"] = round(a16, 3)
+        out["frac_matrix_fp16"] = round(a16 / PEAK_FP16_MATRIX_TFLOPS, 4)
     if "VALUBusy" in c:
         out["valu_busy_rocprof_pct"] = c["VALUBusy"]
     return out
@@ -409,7 +416,8 @@ def roofline_entry(cfg, precision, evals, flop, kernel_ms, f_act):
     (betatron workload only; see executed_roofline).  ``algorithmic``: the
     reference integrand's flop count per evaluation times the evaluations,
     which exceeds the peak because this kernel shares the omega-independent
-    work, rotates instead of taking every sin/cos and skips filtered steps."""
+    work, factors the phases of a linear grid (the sums then run on the matrix
+    cores) and skips filtered steps."""
     kind = "f64" if precision == "double" else "split"
     ex = executed_roofline(kind, kernel_ms) if cfg == 2 else None
     alg = evals * flop / (kernel_ms * 1e-3) / 1e12
@@ -513,11 +521,11 @@ def bench_adjoint(args):
         ex = executed_roofline(kind, ms_bwd, ADJOINT_COUNTERS_FILE)
         res[prec] = {"ms_fwd_bwd": round(ms, 2), "ms_forward": round(ms - ms_bwd, 2), "ms_backward": round(ms_bwd, 2),
                      "G_evals_per_s_fwd_equiv": round(evals / (ms * 1e-3) / 1e9, 2),
-                     "roofline_backward": {"bound": "valu", "kernel": "k_adjoint (transpose sweep)",
+                     "roofline_backward": {"bound": "valu", "kernel": "transpose sweep",
                                            "achieved": ex["achieved_fp32_equiv"] if ex else None,
                                            "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                                            "frac": ex["frac"] if ex else None, "executed": ex,
-                                           "basis": "issued lane-flops of k_adjoint per backward from the counter "
+                                           "basis": "issued lane-flops of the transpose sweep per backward from the counter "
                                                     "totals in profiles/adjoint_betatron_counters.md over this "
                                                     "run's backward time (HIP events around loss.backward(); "
                                                     "includes the slab reduction and the loss's own gradient)"}}

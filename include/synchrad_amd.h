@@ -235,7 +235,9 @@ int sr_spectrum_batch_noalloc(const sr_tracks *tracks, const sr_grid *grid, cons
  * number of direction groups (0 = chosen); opts.waves_per_block the block size
  * of the transpose sweep (threads = steps).  The workspace holds the group
  * slabs, the particles' complex fields for a chunk of particles (at most
- * ~2 GiB; larger batches are processed chunk by chunk) and the step data.
+ * ~2 GiB; larger batches are processed chunk by chunk), the step data and, for
+ * SR_PREC_SPLIT on linear grids, coefficient tables (~256 MiB, one direction of
+ * the chunk's particles at least).
  */
 int sr_far_adjoint_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid, const sr_opts *opts,
                                    size_t *bytes);

@@ -57,9 +57,11 @@ MAX_REPS = 50
 
 def candidates(mode: str, precision: str, uniform: bool, n_omega: int) -> List[engine.Tuning]:
     """Plans worth timing: FP64 sweeps directly with 1 or 2 omegas per thread;
-    split precision uses the recurrence on linear grids (measured faster there
-    than every direct plan) and the direct sweep otherwise.  Blocks whose
-    omega run would leave more than a quarter of their lanes idle are left out."""
+    split precision uses matrix products on linear grids ("recurrence": measured
+    faster there than every direct plan; M = 4 allows tiles of up to 512 omegas,
+    2 up to 256, and the waves share a tile's steps) and the direct sweep
+    otherwise.  Blocks whose omega run would leave more than a quarter of their
+    lanes idle are left out."""
     T = engine.Tuning
     if engine.PRECISIONS[precision] == _abi.SR_PREC_F64:
         pairs = [("direct", m, w) for m in (1, 2) for w in (1, 2, 4)]

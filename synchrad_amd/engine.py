@@ -366,7 +366,7 @@ class DeviceGrid:
 def uniform_step(w: np.ndarray, rtol: float = 1e-14) -> float:
     """The constant step of ``w`` if every sample lies within ``rtol*max|w|``
     of w[0] + i*step (linear grids built by np.r_/linspace do), else 0.  The
-    recurrence sweep uses it; the bound keeps its phase error below
+    factored sweeps use it; the bound keeps their phase error below
     rtol*max|omega*tau|."""
     n = w.size
     if n < 2:
