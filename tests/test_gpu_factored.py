@@ -141,3 +141,11 @@ def test_small_component_keeps_its_accuracy():
         # BOUND is relative to sum |A_s|; on the undulator line the sum itself is
         # at least a tenth of it in the 2-norm over these omegas
         assert err <= 10 * BOUND * size
+
+
+@pytest.mark.parametrize("n_steps", [1007, 1008, 1009])
+@pytest.mark.parametrize("kind,n_omega", [("up", 2), ("up", 24), ("down", 33), ("cross", 64)])
+def test_small_grids_of_long_tracks(kind, n_omega, n_steps):
+    """Grids of at most one wave's frequencies, at the track length where they take the
+    factored tiles; four waves share the steps."""
+    test_far_edges(kind, n_omega, n_steps, 0, 0)
