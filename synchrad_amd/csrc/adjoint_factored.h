@@ -563,12 +563,14 @@ k_adjoint_factored(const AParams p) {
             float2 ph;
             sincos_rev(s_alpha[g] * tau, &ph.y, &ph.x);
             const bool more = cut_r > 16;
-            const float low = mine && (more != up) ? 1.f : 0.f, high = mine && (more == up) ? 1.f : 0.f;
-            const float sgn = more ? -1.f : 1.f;
+            const bool low = mine && more != up, high = mine && more == up;
+            const float cs = more ? -ph.x : ph.x, sn = more ? -ph.y : ph.y;
             const uint32_t from = mine ? (uint32_t)(more ? cut_r - 16 : 16 - cut_r) : 16u;
             sr::wave_sync();
             s_msk[lane] = from | (from << 16);
-            s_al[lane] = make_float4(sgn * low * ph.x, sgn * low * ph.y, sgn * high * ph.x, sgn * high * ph.y);
+            // (selected, not multiplied by zero: the phase of a step at a position that is
+            // not finite stays out of its sums, as the step does)
+            s_al[lane] = make_float4(low ? cs : 0.f, low ? sn : 0.f, high ? cs : 0.f, high ? sn : 0.f);
             sr::wave_sync();
 #pragma unroll
             for (int set = 0; set < NSET; set++) {

@@ -93,6 +93,18 @@ def test_coefficients_that_are_not_finite_stay_with_the_steps_that_keep_them():
         assert torch.equal(torch.isfinite(a[c]), torch.isfinite(b[c]))
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("comp", ["total", "cartesian"])
+def test_positions_that_are_not_finite_stay_out(comp, bad):
+    """A sample at such a position keeps no frequency (nor does the one after it), so its
+    gradients are zero, as in the FP64 path, also where its wave's other steps cut groups."""
+    wl = workloads.config2(n_particles=1, n_steps=1100, grid=(100, 4, 3))
+    axes = dict(wl.axes, omega=np.linspace(0.0, 6.0 * wl.axes["omega"][-1], 100))
+    track = [np.array(c) for c in wl.track_list()[0][:6]]
+    track[0][[200, 777]] = bad
+    _check(wl, axes, comp, tracks=[track + [1.0, 0]])
+
+
 def test_tables_of_several_launches():
     """More tables than fit at once: 90 electrons, 32 x 32 directions, 128 frequencies."""
     wl = workloads.config2(n_particles=90, n_steps=390, grid=(128, 32, 32))
