@@ -3,7 +3,7 @@ steps, synchrad_amd/csrc/factored.h) against the CPU FP64 oracle, at the sizes
 where it can go wrong: omega counts around the 32-omega groups and the 128-,
 256- and 512-omega tiles, step counts around the 63-step stretches and the
 32-step products, every order of the omegas (descending, negative, through
-zero), and tracks whose amplitude jumps or vanishes.
+zero), steps that keep part of the frequencies (far and near), and tracks whose amplitude jumps or vanishes.
 
 Bound, per complex field component: each term A_s e^{i phase} passes through at
 most eleven FP32-level roundings (two phasor factors and their product on each
@@ -74,27 +74,69 @@ def test_far_edges(kind, n_omega, n_steps, M, W):
     assert worst <= BOUND
 
 
-@pytest.mark.parametrize("n_omega,n_steps", [(64, 65), (130, 500), (300, 127)])
-def test_near_edges(n_omega, n_steps):
-    wl = workloads.config4(n_particles=1)
-    tr = [[c[:n_steps] for c in wl.track_list()[0][:6]] + [1.0, 0]]
-    axes = {"omega": np.linspace(wl.axes["omega"][0], wl.axes["omega"][-1], n_omega),
-            "radius": np.linspace(0.0, 0.07, 3), "phi": np.array([0.0, 2.0])}
-    dt, L = wl.batch.dt, wl.L_screen
+def _check_near(wl, tr, axes, dt, tuning=None):
+    """The complex field within BOUND of sum_s |v2| + |omega| |v1| at each screen point."""
+    L = wl.L_screen
     ref = oracle.spectrum("near", "cartesian_complex", tr, axes, dt, L_screen=L)
-    got = _run("near", "cartesian_complex", tr, axes, dt, L_screen=L)
-    # |v2| + omega |v1| summed over the steps at each screen point
+    got = _run("near", "cartesian_complex", tr, axes, dt, tuning, L_screen=L)
     x, y, z, ux, uy, uz = tr[0][:6]
     b = (np.stack([ux, uy, uz], 1) / np.sqrt(1 + ux ** 2 + uy ** 2 + uz ** 2)[:, None])[:-1]
-    om = 2 * np.pi * axes["omega"]
+    om = np.abs(2 * np.pi * axes["omega"])
+    worst = 0.0
     for i, r in enumerate(axes["radius"]):
         for j, ph in enumerate(axes["phi"]):
             d = np.array([r * np.cos(ph), r * np.sin(ph), L]) - np.stack([x, y, z], 1)[:-1]
             R = np.linalg.norm(d, axis=1)
             n = d / R[:, None]
             total = dt * ((1 / R ** 2).sum() + om * (np.linalg.norm(b - n, axis=1) / R).sum())
-            for k in ref:
-                assert np.max(np.abs(got[k] - ref[k])[0, :, i, j] / total) <= BOUND, (k, i, j)
+            worst = max(worst, *(float(np.max(np.abs(got[k] - ref[k])[0, :, i, j] / total)) for k in ref))
+    print(f"{axes['omega'].size} omegas {x.size} steps: {worst:.2e} of the sum of the terms", flush=True)
+    assert worst <= BOUND
+
+
+@pytest.mark.parametrize("n_omega,n_steps", [(64, 65), (130, 500), (300, 127)])
+def test_near_edges(n_omega, n_steps):
+    """Grids that every step keeps whole (past the first, which keeps none)."""
+    wl = workloads.config4(n_particles=1)
+    tr = [[c[:n_steps] for c in wl.track_list()[0][:6]] + [1.0, 0]]
+    axes = {"omega": np.linspace(wl.axes["omega"][0], wl.axes["omega"][-1], n_omega),
+            "radius": np.linspace(0.0, 0.07, 3), "phi": np.array([0.0, 2.0])}
+    _check_near(wl, tr, axes, wl.batch.dt)
+
+
+def _near_kept(wl, tr, axes, dt):
+    """How many frequencies each step keeps at each screen point, those of smallest |omega|."""
+    x, y, z = tr[0][:3]
+    om = np.sort(np.abs(axes["omega"]))
+    kept = []
+    for r in axes["radius"]:
+        for ph in axes["phi"]:
+            R = np.sqrt((r * np.cos(ph) - x) ** 2 + (r * np.sin(ph) - y) ** 2 + (wl.L_screen - z) ** 2)
+            tau = np.arange(x.size) * dt + R
+            kept.append(np.searchsorted(om, 0.5 / np.abs(np.diff(tau[:-1]))))
+    return np.concatenate(kept)
+
+
+@pytest.mark.parametrize("kind,n_omega,n_steps,every,M,W", [
+    ("up", 31, 300, 1, 0, 1), ("up", 33, 300, 1, 0, 2), ("up", 64, 500, 1, 0, 4), ("up", 65, 500, 3, 2, 1),
+    ("up", 129, 700, 1, 0, 0), ("up", 300, 400, 3, 4, 2), ("down", 33, 300, 3, 0, 1), ("down", 129, 700, 1, 0, 4),
+    ("negative", 100, 400, 1, 2, 2), ("cross", 65, 500, 1, 0, 0), ("cross down", 260, 500, 3, 0, 1)])
+def test_near_cut_steps(kind, n_omega, n_steps, every, M, W):
+    """Frequencies across the steps' thresholds, in every order of the grid: steps that
+    keep part of a group, in its lower and in its upper half."""
+    wl = workloads.config4(n_particles=1)
+    dt = every * wl.batch.dt
+    tr = [[c[::every][:n_steps] for c in wl.track_list()[0][:6]] + [1.0, 0]]
+    lo, hi = wl.axes["omega"][0], 7.3 * wl.axes["omega"][-1]
+    omega = {"up": np.linspace(lo, hi, n_omega), "down": np.linspace(hi, lo, n_omega),
+             "negative": np.linspace(-hi, -lo, n_omega), "cross": np.linspace(-0.37 * hi, hi, n_omega),
+             "cross down": np.linspace(0.61 * hi, -hi, n_omega)}[kind]
+    axes = {"omega": omega, "radius": np.linspace(0.0, 0.071, 3), "phi": np.array([0.3, 2.1])}
+    if not kind.startswith("cross"):
+        kept = _near_kept(wl, tr, axes, dt)
+        part = kept[(kept > 0) & (kept < n_omega)] % 32
+        assert ((part > 0) & (part <= 16)).sum() > 20 and (part > 16).sum() > 20
+    _check_near(wl, tr, axes, dt, engine.Tuning(omega_per_lane=M, waves_per_block=W))
 
 
 def test_amplitude_range_and_snapshots():
