@@ -376,6 +376,7 @@ k_factored(const KParams p) {
           auto sweep_block = [&](auto type) {
             constexpr int q = decltype(type)::value;
             constexpr bool CUT = q != 0;
+            wave_sync();   // the block before has read its factors
             const Lanes L = kHoist ? held : lanes();
             const int at = head[q] + 8 * L.kg;
             // ---- the block's factors: lanes 0..31 the columns' of step l, lanes

@@ -191,3 +191,12 @@ def test_small_grids_of_long_tracks(kind, n_omega, n_steps):
     """Grids of at most one wave's frequencies, at the track length where they take the
     factored tiles; four waves share the steps."""
     test_far_edges(kind, n_omega, n_steps, 0, 0)
+
+
+@pytest.mark.parametrize("n_steps", [64, 95, 96, 126, 127, 158, 190, 253])
+@pytest.mark.parametrize("n_omega", [100, 200, 400])
+def test_blocks_in_succession(n_omega, n_steps):
+    """One wave sweeping one, two and three blocks of steps with nothing between them:
+    two blocks of one queue, and at the track's end the rest of every queue, each
+    rewriting the factors that the block before has read."""
+    test_far_edges("up", n_omega, n_steps, 0, 1)
