@@ -222,12 +222,14 @@ struct WavesPerEU {
 };
 
 // PRE: the step data come from the pre-pass records (batch calls); without
-// them (the per-particle and no-allocation calls) the stage forms them from u
-template <int MODE, int PREC, int M, bool PRE>
-__global__ void __launch_bounds__(PREC == SR_PREC_F64 ? kWave * kMaxParts : kMaxT)
+// them (the per-particle and no-allocation calls) the stage forms them from u.
+// PARTS (FP64): several groups of threads share a tile's steps (KParams::parts)
+template <int MODE, int PREC, int M, bool PRE, bool PARTS>
+__global__ void __launch_bounds__(PARTS ? kWave * kMaxParts : kMaxT)
 __attribute__((amdgpu_waves_per_eu(WavesPerEU<MODE, PREC, M>::value)))
 k_spectrum(const KParams p) {
   static_assert(PREC == SR_PREC_SPLIT || M <= 2, "the FP64 sweep holds one or two omegas per thread");
+  static_assert(PREC == SR_PREC_F64 || !PARTS, "the split sweep has one group of threads");
   using Amp = typename std::conditional<PREC == SR_PREC_SPLIT, float, double>::type;
   constexpr bool kSplit = (PREC == SR_PREC_SPLIT);
   // amplitude words per step.  Far: A is perpendicular to n
@@ -237,7 +239,7 @@ k_spectrum(const KParams p) {
   constexpr int NA = amp_words<MODE, PREC>();
   constexpr int NC = (MODE == SR_MODE_FAR) ? 2 * NA : 6;   // real accumulators per omega
   constexpr int NP = (MODE == SR_MODE_FAR) ? NC : 12;      // split register partials per omega
-  constexpr int kMaxW = kSplit ? kMaxT / kWave : kMaxParts;   // waves per block
+  constexpr int kMaxW = PARTS ? kMaxParts : kMaxT / kWave;    // waves per block
 
   extern __shared__ __align__(16) char s_dyn_raw[];
   // FP64 sin/cos table (sincos_table) and the largest |omega| of the grid
@@ -246,11 +248,11 @@ k_spectrum(const KParams p) {
   __shared__ double s_wmax[kTab ? kMaxW : 1];
   __shared__ int s_vote[kMaxW];   // per-wave votes of a block-wide any/all
 
-  // the block's groups of T threads (FP64; the split sweep has one) each hold the
-  // tile's omegas and sweep a part of every track; their sums meet at the records
-  const int P = kSplit ? 1 : p.parts;
-  const int T = kSplit ? (int)blockDim.x : (int)blockDim.x / P;
-  const int grp = kSplit ? 0 : uni((int)threadIdx.x / T);
+  // the block's groups of T threads each hold the tile's omegas and sweep a part of
+  // every track; their sums meet at the records
+  const int P = PARTS ? p.parts : 1;
+  const int T = PARTS ? (int)blockDim.x / P : (int)blockDim.x;
+  const int grp = PARTS ? uni((int)threadIdx.x / T) : 0;
   const int tid = (int)threadIdx.x - grp * T;
   const int W = T / kWave;
   const int wv = uni(tid / kWave);   // wave-uniform: its derived indices stay scalar
@@ -610,23 +612,8 @@ k_spectrum(const KParams p) {
         return time + sqrt(rx * rx + ry * ry + rz * rz);
       };
 
-      // the steps up to each snapshot record, [done, seg_hi), cut into the groups'
-      // parts of `per` steps; the records after the last active step (global
-      // it_range mode) see the final sums
-      int64_t done = 0;
-      while (cur.next >= 0) {
-      const int64_t seg_hi = max(done, min(cur.next + 1, n_act));
-      const int64_t per = (seg_hi - done + P - 1) / P;
-      const int64_t lo = min(done + grp * per, seg_hi), hi = min(lo + per, seg_hi);
-      if (!kSplit) {
-        // FP64: the phase before the part's first step (phase_{-1} = 0)
-        const double before = lo > 0 ? tau_at(lo - 1) : 0.0;
-#pragma unroll
-        for (int k = 0; k < M; k++) prev[k] = om[k] * before;
-      }
-      for (int64_t it = 0; it < per; it += T) {
-        const int64_t t0 = lo + it;
-        const int cnt = uni((int)max((int64_t)0, min((int64_t)T, hi - t0)));
+      // stages the group's steps [t0, t0 + cnt), cnt <= T
+      auto stage_tile = [&](int64_t t0, int cnt) {
         __syncthreads();  // previous tile fully consumed
         int st_wide = 0;
         if (tid < cnt) {
@@ -736,37 +723,71 @@ k_spectrum(const KParams p) {
         } else {
           __syncthreads();
         }
+      };
+      auto emit_next = [&]() {
+        if (grp == 0) emit(cur.slot);
+        const int64_t last = cur.next;
+        cur.slot++;
+        cur.advance(pt, p.n_snaps, last);
+      };
 
-        // ---- sweep, split at snapshot records falling inside the tile ----
-        int j = 0;
-        direct_sweep(j, cnt);
-        kahan_fold();
-      }
-      done = seg_hi;
-      if (!kSplit && P > 1) {
-        // the other groups' sums so far go to the first group, one word at a time
+      if constexpr (PARTS) {
+        // the steps up to each snapshot record, [done, seg_hi), cut into the groups'
+        // parts of `per` steps (P is a power of two); the records after the last active
+        // step (global it_range mode) see the final sums
+        int64_t done = 0;
+        while (cur.next >= 0) {
+          const int64_t seg_hi = max(done, min(cur.next + 1, n_act));
+          const int64_t per = (seg_hi - done + P - 1) >> __builtin_ctz(P);
+          const int64_t lo = min(done + grp * per, seg_hi), hi = min(lo + per, seg_hi);
+          // the phase before the part's first step (phase_{-1} = 0)
+          const double before = lo > 0 ? tau_at(lo - 1) : 0.0;
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-          __syncthreads();
-          if (grp > 0) {
+          for (int k = 0; k < M; k++) prev[k] = om[k] * before;
+          for (int64_t it = 0; it < per; it += T) {
+            const int cnt = uni((int)max((int64_t)0, min((int64_t)T, hi - lo - it)));
+            stage_tile(lo + it, cnt);
+            int j = 0;
+            direct_sweep(j, cnt);
+          }
+          done = seg_hi;
+          // the other groups' sums so far go to the first group, one word at a time
 #pragma unroll
-            for (int k = 0; k < M; k++) {
-              s_sum[((grp - 1) * M + k) * T] = fs[k][c];
-              fs[k][c] = 0.0;
+          for (int c = 0; c < NC; c++) {
+            __syncthreads();
+            if (grp > 0) {
+#pragma unroll
+              for (int k = 0; k < M; k++) {
+                s_sum[((grp - 1) * M + k) * T] = fs[k][c];
+                fs[k][c] = 0.0;
+              }
+            }
+            __syncthreads();
+            if (grp == 0) {
+              for (int q1 = 0; q1 < P - 1; q1++)
+#pragma unroll
+                for (int k = 0; k < M; k++) fs[k][c] += s_sum[(q1 * M + k) * T];
             }
           }
-          __syncthreads();
-          if (grp == 0) {
-            for (int q1 = 0; q1 < P - 1; q1++)
-#pragma unroll
-              for (int k = 0; k < M; k++) fs[k][c] += s_sum[(q1 * M + k) * T];
+          emit_next();
+        }
+      } else {
+        // tiles of T steps, their sweep split at the records (one electron's 1600 steps on
+        // 256 x 32 x 32, 100 and 400 records: log grid 377 and 1178 us, FP64 534 and 1123;
+        // with a tile staged anew after each record 411 and 1309, 754 and 2359)
+        for (int64_t t0 = 0; t0 < n_act && cur.next >= 0; t0 += T) {
+          const int cnt = uni((int)min((int64_t)T, n_act - t0));
+          stage_tile(t0, cnt);
+          int j = 0;
+          while (j < cnt && cur.next >= 0) {
+            const bool here = cur.next < t0 + cnt;
+            direct_sweep(j, uni(here ? (int)(cur.next - t0) + 1 : cnt));
+            kahan_fold();
+            if (here) emit_next();
           }
         }
-      }
-      if (grp == 0) emit(cur.slot);
-      const int64_t last = cur.next;
-      cur.slot++;
-      cur.advance(pt, p.n_snaps, last);
+        // records after the last active step (global it_range mode) see the final sums
+        while (cur.next >= 0) emit_next();
       }
     }
     if (late_s(p.acc_lds) && grp == 0) {
@@ -987,6 +1008,12 @@ double factored_cost(bool far, int groups) {
   return 9.75;
 }
 
+// FP64: steps up to a record that each group of threads has at least.  The groups meet at
+// every record: one electron's 1600 steps on 32 x 4 x 4 with a record every 80, 32 and 16
+// steps 110, 216, 308 us at 16 (4, 2, 1 groups), 108, 192, 330 at 8, 152, 276, 308 at 32;
+// 8 electrons on 100 x 12 x 12 297, 385, 459, at 8 352, 385, 546
+constexpr int64_t kPartSteps = 16;
+
 // omegas of one tile
 int64_t tile_run(const Plan &pl) {
   return pl.sweep == SWEEP_REC ? 32 * (int64_t)pl.groups : (int64_t)kWave * pl.waves * pl.M;
@@ -1003,6 +1030,8 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   Plan pl;
   const int64_t n_om = g.n_omega;
   const int64_t n_dir = (int64_t)g.n_theta * g.n_phi;
+  // steps up to a record
+  const int64_t record_steps = mean_steps / std::max<int64_t>(1, n_snaps);
   // AUTO: the factored tiles for split spectra on linear grids, except far-field
   // grids of at most one 64-omega wave: there the direct sweep's sine per omega
   // costs no more than forming the factors (32 betatron electrons on 64 x 32 x 32:
@@ -1017,10 +1046,11 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
        (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave || (mean_steps >= 1008 && spread < 2048)))))
     pl.sweep = SWEEP_REC;
   // FP64: groups of threads that may share a tile's steps: blocks of at most
-  // kMaxParts waves, two staged tiles of steps for each
+  // kMaxParts waves, two staged tiles of steps for each, and of the steps up to a
+  // record kPartSteps
   auto part_limit = [&](int w) -> int64_t {
     if (o.precision != SR_PREC_F64) return 1;
-    return std::max<int64_t>(1, std::min<int64_t>(kMaxParts / w, mean_steps / (2 * kWave * w)));
+    return std::max<int64_t>(1, std::min<int64_t>({kMaxParts / w, mean_steps / (2 * kWave * w), record_steps / kPartSteps}));
   };
   int64_t chunks;
   if (pl.sweep == SWEEP_REC) {
@@ -1069,9 +1099,10 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
         const int64_t c = (n_om + run - 1) / run;
         const double eff = (double)n_om / (double)(c * run);
         if (eff < 0.75) continue;
-        // M = 2 measured fastest, also against twice the waves (256 omegas FP64: one
-        // undulator electron 0.38 ms at 2 x 2 waves, 0.42 at 1 x 4)
-        const double mpref = (m == 2) ? 0.03 : 0.0;
+        // M = 2 measured fastest, with groups of threads also against twice the waves
+        // (256 omegas FP64: one undulator electron 0.38 ms at 2 x 2 waves, 0.42 at 1 x 4;
+        // without them 100 omegas on 12 x 12, 200 records: 0.41 ms at 1 x 2, 0.74 at 2 x 1)
+        const double mpref = (m == 2) ? (part_limit(w) > 1 ? 0.03 : 0.02) : 0.0;
         // launches too small to fill the GPU (one particle: no slices to add
         // waves) prefer the plan with the most waves: 256 CUs hold ~8K waves
         const double fill = std::min(1.0, (double)(c * n_dir * w * part_limit(w) *
@@ -1126,21 +1157,20 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   pl.parts = 1;
   while (2 * pl.parts <= part_limit(pl.waves) && base_waves * s * pl.parts < 4096) pl.parts *= 2;
   pl.blocks = chunks * n_dir * s;
-  (void)n_snaps;
   return pl;
 }
 
-template <int MODE, int PREC, int M>
+template <int MODE, int PREC, int M, bool PARTS = false>
 hipError_t launch_t(const KParams &kp, int64_t grid, int threads, hipStream_t st) {
   const int T = threads / kp.parts;
   const size_t lds = kp.parts * stage_lds_bytes<MODE, PREC>(T) +
                      ((PREC == SR_PREC_SPLIT) ? kahan_lds_bytes<MODE, M>(T) : 0) +
                      (kp.acc_lds ? acc_lds_bytes<M>(T) : 0) + (kp.parts - 1) * acc_lds_bytes<M>(T);
   if (kp.pre)
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, true>), dim3((unsigned)grid), dim3(threads), lds, st,
+    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, true, PARTS>), dim3((unsigned)grid), dim3(threads), lds, st,
                        kp);
   else
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, false>), dim3((unsigned)grid), dim3(threads), lds, st,
+    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, false, PARTS>), dim3((unsigned)grid), dim3(threads), lds, st,
                        kp);
   return hipGetLastError();
 }
@@ -1159,6 +1189,9 @@ template <int MODE>
 hipError_t launch_mode(const Plan &pl, int prec, const KParams &kp, int64_t grid, int threads,
                        hipStream_t st) {
   if (prec == SR_PREC_F64) {
+    if (pl.parts > 1)
+      return pl.M == 2 ? launch_t<MODE, SR_PREC_F64, 2, true>(kp, grid, threads, st)
+                       : launch_t<MODE, SR_PREC_F64, 1, true>(kp, grid, threads, st);
     if (pl.M == 2) return launch_t<MODE, SR_PREC_F64, 2>(kp, grid, threads, st);
     return launch_t<MODE, SR_PREC_F64, 1>(kp, grid, threads, st);
   }

@@ -38,6 +38,33 @@ def test_parts_and_snapshots(it_range, nSnaps):
     check(got, ref, "double", f"snapshots {it_range}")
 
 
+@pytest.mark.parametrize("precision,W", [("double", 0), ("double", 4), ("float", 1), ("float", 4)])
+@pytest.mark.parametrize("it_range,nSnaps", [((0, 1500), 11), ((0, 1500), 60), ((0, 1500), 375), ((200, 900), 700), (None, 300)])
+def test_many_records(precision, W, it_range, nSnaps):
+    """Records at every distance, down to one at each step: parts of the steps between
+    records, and records inside a staged tile, on its last step and after the last active
+    one (FP64, and the split direct sweep on a logarithmic grid)."""
+    wl = workloads.config2(n_particles=2, n_steps=1400, grid=(40, 3, 2))
+    axes = dict(wl.axes)
+    if precision == "float":
+        axes["omega"] = np.geomspace(axes["omega"][0], axes["omega"][-1], 40)
+    tr = [[c[:n] for c in t[:6]] + [t[6], its] for t, n, its in zip(wl.track_list(), (1400, 301), (0, 150))]
+    ref = oracle.spectrum("far", "total", tr, axes, wl.batch.dt, it_range=it_range, nSnaps=nSnaps)
+    got = gpu_spectrum(tr, axes, wl.batch.dt, precision=precision, it_range=it_range, nSnaps=nSnaps,
+                       tuning=engine.Tuning(waves_per_block=W))
+    check(got, ref, precision, f"{nSnaps} records")
+
+
+@pytest.mark.parametrize("nSnaps", [7, 40, 350])
+def test_near_many_records(nSnaps):
+    wl = workloads.config4(n_particles=1)
+    tr = [[c[:700] for c in wl.track_list()[0][:6]] + [1.0, 0]]
+    axes = dict(omega=wl.axes["omega"][:70], radius=wl.axes["radius"][::24], phi=wl.axes["phi"][::32])
+    ref = oracle.spectrum("near", "cartesian_complex", tr, axes, wl.batch.dt, L_screen=wl.L_screen, nSnaps=nSnaps)
+    got = gpu_spectrum(tr, axes, wl.batch.dt, mode="near", comp="cartesian_complex", L_screen=wl.L_screen, nSnaps=nSnaps)
+    check(got, ref, "double", f"near {nSnaps} records")
+
+
 @pytest.mark.parametrize("n_steps", [700, 2300])
 def test_near_parts(n_steps):
     """The longer track takes the largest block, 16 waves: its LDS is past 64 KiB."""
