@@ -223,13 +223,16 @@ struct WavesPerEU {
 
 // PRE: the step data come from the pre-pass records (batch calls); without
 // them (the per-particle and no-allocation calls) the stage forms them from u.
-// PARTS (FP64): several groups of threads share a tile's steps (KParams::parts)
-template <int MODE, int PREC, int M, bool PRE, bool PARTS>
-__global__ void __launch_bounds__(PARTS ? kWave * kMaxParts : kMaxT)
+// RECORDS: the sweep of a staged tile is split at the snapshot records in it, for launches
+// with several and one group of threads; else the steps up to a record are staged by
+// themselves, in the groups' parts (with one record the shorter code: 120 tracks of up to
+// 20000 steps on a 256 x 32 x 32 log grid 36.7 ms against 37.1, FP64 24 x 4000 17.0 against
+// 17.4)
+template <int MODE, int PREC, int M, bool PRE, bool RECORDS>
+__global__ void __launch_bounds__(PREC == SR_PREC_F64 && !RECORDS ? kWave * kMaxParts : kMaxT)
 __attribute__((amdgpu_waves_per_eu(WavesPerEU<MODE, PREC, M>::value)))
 k_spectrum(const KParams p) {
   static_assert(PREC == SR_PREC_SPLIT || M <= 2, "the FP64 sweep holds one or two omegas per thread");
-  static_assert(PREC == SR_PREC_F64 || !PARTS, "the split sweep has one group of threads");
   using Amp = typename std::conditional<PREC == SR_PREC_SPLIT, float, double>::type;
   constexpr bool kSplit = (PREC == SR_PREC_SPLIT);
   // amplitude words per step.  Far: A is perpendicular to n
@@ -239,7 +242,8 @@ k_spectrum(const KParams p) {
   constexpr int NA = amp_words<MODE, PREC>();
   constexpr int NC = (MODE == SR_MODE_FAR) ? 2 * NA : 6;   // real accumulators per omega
   constexpr int NP = (MODE == SR_MODE_FAR) ? NC : 12;      // split register partials per omega
-  constexpr int kMaxW = PARTS ? kMaxParts : kMaxT / kWave;    // waves per block
+  constexpr bool kParts = !kSplit && !RECORDS;             // several groups of threads
+  constexpr int kMaxW = kParts ? kMaxParts : kMaxT / kWave;   // waves per block
 
   extern __shared__ __align__(16) char s_dyn_raw[];
   // FP64 sin/cos table (sincos_table) and the largest |omega| of the grid
@@ -250,9 +254,9 @@ k_spectrum(const KParams p) {
 
   // the block's groups of T threads each hold the tile's omegas and sweep a part of
   // every track; their sums meet at the records
-  const int P = PARTS ? p.parts : 1;
-  const int T = PARTS ? (int)blockDim.x / P : (int)blockDim.x;
-  const int grp = PARTS ? uni((int)threadIdx.x / T) : 0;
+  const int P = kParts ? p.parts : 1;
+  const int T = kParts ? (int)blockDim.x / P : (int)blockDim.x;
+  const int grp = kParts ? uni((int)threadIdx.x / T) : 0;
   const int tid = (int)threadIdx.x - grp * T;
   const int W = T / kWave;
   const int wv = uni(tid / kWave);   // wave-uniform: its derived indices stay scalar
@@ -731,7 +735,7 @@ k_spectrum(const KParams p) {
         cur.advance(pt, p.n_snaps, last);
       };
 
-      if constexpr (PARTS) {
+      if constexpr (!RECORDS) {
         // the steps up to each snapshot record, [done, seg_hi), cut into the groups'
         // parts of `per` steps (P is a power of two); the records after the last active
         // step (global it_range mode) see the final sums
@@ -740,33 +744,38 @@ k_spectrum(const KParams p) {
           const int64_t seg_hi = max(done, min(cur.next + 1, n_act));
           const int64_t per = (seg_hi - done + P - 1) >> __builtin_ctz(P);
           const int64_t lo = min(done + grp * per, seg_hi), hi = min(lo + per, seg_hi);
-          // the phase before the part's first step (phase_{-1} = 0)
-          const double before = lo > 0 ? tau_at(lo - 1) : 0.0;
+          if (!kSplit) {
+            // FP64: the phase before the part's first step (phase_{-1} = 0)
+            const double before = lo > 0 ? tau_at(lo - 1) : 0.0;
 #pragma unroll
-          for (int k = 0; k < M; k++) prev[k] = om[k] * before;
+            for (int k = 0; k < M; k++) prev[k] = om[k] * before;
+          }
           for (int64_t it = 0; it < per; it += T) {
             const int cnt = uni((int)max((int64_t)0, min((int64_t)T, hi - lo - it)));
             stage_tile(lo + it, cnt);
             int j = 0;
             direct_sweep(j, cnt);
+            kahan_fold();
           }
           done = seg_hi;
-          // the other groups' sums so far go to the first group, one word at a time
+          if (kParts && P > 1) {
+            // the other groups' sums so far go to the first group, one word at a time
 #pragma unroll
-          for (int c = 0; c < NC; c++) {
-            __syncthreads();
-            if (grp > 0) {
+            for (int c = 0; c < NC; c++) {
+              __syncthreads();
+              if (grp > 0) {
 #pragma unroll
-              for (int k = 0; k < M; k++) {
-                s_sum[((grp - 1) * M + k) * T] = fs[k][c];
-                fs[k][c] = 0.0;
+                for (int k = 0; k < M; k++) {
+                  s_sum[((grp - 1) * M + k) * T] = fs[k][c];
+                  fs[k][c] = 0.0;
+                }
               }
-            }
-            __syncthreads();
-            if (grp == 0) {
-              for (int q1 = 0; q1 < P - 1; q1++)
+              __syncthreads();
+              if (grp == 0) {
+                for (int q1 = 0; q1 < P - 1; q1++)
 #pragma unroll
-                for (int k = 0; k < M; k++) fs[k][c] += s_sum[(q1 * M + k) * T];
+                  for (int k = 0; k < M; k++) fs[k][c] += s_sum[(q1 * M + k) * T];
+              }
             }
           }
           emit_next();
@@ -1160,18 +1169,20 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   return pl;
 }
 
-template <int MODE, int PREC, int M, bool PARTS = false>
+template <int MODE, int PREC, int M>
 hipError_t launch_t(const KParams &kp, int64_t grid, int threads, hipStream_t st) {
   const int T = threads / kp.parts;
   const size_t lds = kp.parts * stage_lds_bytes<MODE, PREC>(T) +
                      ((PREC == SR_PREC_SPLIT) ? kahan_lds_bytes<MODE, M>(T) : 0) +
                      (kp.acc_lds ? acc_lds_bytes<M>(T) : 0) + (kp.parts - 1) * acc_lds_bytes<M>(T);
-  if (kp.pre)
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, true, PARTS>), dim3((unsigned)grid), dim3(threads), lds, st,
-                       kp);
-  else
-    hipLaunchKernelGGL((k_spectrum<MODE, PREC, M, false, PARTS>), dim3((unsigned)grid), dim3(threads), lds, st,
-                       kp);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(threads), lds, st, kp); };
+  if (kp.n_snaps > 1 && kp.parts == 1) {
+    if (kp.pre) launch(k_spectrum<MODE, PREC, M, true, true>);
+    else launch(k_spectrum<MODE, PREC, M, false, true>);
+  } else {
+    if (kp.pre) launch(k_spectrum<MODE, PREC, M, true, false>);
+    else launch(k_spectrum<MODE, PREC, M, false, false>);
+  }
   return hipGetLastError();
 }
 
@@ -1189,9 +1200,6 @@ template <int MODE>
 hipError_t launch_mode(const Plan &pl, int prec, const KParams &kp, int64_t grid, int threads,
                        hipStream_t st) {
   if (prec == SR_PREC_F64) {
-    if (pl.parts > 1)
-      return pl.M == 2 ? launch_t<MODE, SR_PREC_F64, 2, true>(kp, grid, threads, st)
-                       : launch_t<MODE, SR_PREC_F64, 1, true>(kp, grid, threads, st);
     if (pl.M == 2) return launch_t<MODE, SR_PREC_F64, 2>(kp, grid, threads, st);
     return launch_t<MODE, SR_PREC_F64, 1>(kp, grid, threads, st);
   }
