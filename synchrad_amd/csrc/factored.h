@@ -638,6 +638,16 @@ k_factored(const KParams p) {
                   }
                 }
               }
+              // (nothing swept or queued under the old scales, as at a track's start: they change
+              // here, not by another pass)
+              if (rescale && blocks + fill[0] + fill[1] + fill[2] == 0) {
+#pragma unroll
+                for (int w = 0; w < NW; w++) {
+                  ex[w] = want[w];
+                  af[w] = (float)ldexp(am[w], ex[w]);
+                }
+                rescale = false;
+              }
               if (!rescale) {
                 flush = false;
                 const uint64_t bf = __ballot(K == count);

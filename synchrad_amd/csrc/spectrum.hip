@@ -1039,20 +1039,32 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   Plan pl;
   const int64_t n_om = g.n_omega;
   const int64_t n_dir = (int64_t)g.n_theta * g.n_phi;
+  const bool far = g.mode == SR_MODE_FAR;
+  const int64_t spread = n_dir * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices);
   // steps up to a record
   const int64_t record_steps = mean_steps / std::max<int64_t>(1, n_snaps);
-  // AUTO: the factored tiles for split spectra on linear grids, except far-field
-  // grids of at most one 64-omega wave: there the direct sweep's sine per omega
-  // costs no more than forming the factors (32 betatron electrons on 64 x 32 x 32:
-  // 3.38 ms against 3.62; on 72 omegas 6.8 against 3.6).  Long tracks on too few
-  // directions to fill the GPU take them there too: the direct sweep has no more waves
-  // than tiles, a factored tile's steps are shared by four (one electron x 6000 steps on
-  // 24 x 20 x 4 495 us against 86)
-  const int64_t spread = n_dir * std::min<int64_t>(std::max<int64_t>(n_particles, 1), kMaxSlices);
+  // AUTO: the factored tiles for split spectra on linear grids of more than one 64-omega
+  // wave, from the record length on at which the rest of their queues, the fold and the
+  // waves' meeting at each record are paid for (direct against factored: 1000 betatron
+  // tracks of 32, 64 and 128 steps, 12 x 12 directions: 128 omegas 0.81, 1.02, 1.08 times, 512
+  // 0.99, 1.34, 1.66, complex 256 omegas 0.80, 0.98, 1.20; 24 tracks of 1600 steps with a
+  // record every 64 and 133: 512 omegas 1.05, 1.37, complex 0.65, 0.80, with every
+  // 266 1.21).  On fewer omegas a far-field sine for each costs no more than forming the
+  // factors (32 betatron electrons on 64 x 32 x 32: 3.38 ms against 3.62; on 72 omegas 6.8
+  // against 3.6), but long tracks on too few directions to fill the GPU take the factored
+  // tiles there too: the direct sweep has no more waves than tiles, a factored tile's steps
+  // are shared by four (one electron x 6000 steps on 24 x 20 x 4 495 us against 86; 32 x
+  // 1100 and 4000 on 2 to 64 omegas at a spread of 1920, 1.16 and 1.39 times).  Near field:
+  // the same, and from 256 steps on where the GPU is full (40 tracks on 64 x 16 x 16: 0.78
+  // times at 128 steps, 1.00 at 256, 1.19 at 512)
+  const bool six = o.comp == kCompField || outputs_for(g.mode, o.comp) == 6;
+  const bool full = n_om / ((n_om + 511) / 512) >= 384;   // tiles of 512 omegas, three quarters used
+  bool pays = record_steps >= (six ? 96 : n_snaps > 1 ? 80 : far && full ? 32 : 64);
+  if (n_om <= kWave)
+    pays = pays && (far ? mean_steps >= 1008 && spread < 2048 : record_steps >= 256 || spread < 2048);
   pl.sweep = SWEEP_DIRECT;
   if (o.precision == SR_PREC_SPLIT && g.omega_step != 0.0 &&
-      (o.sweep == SR_SWEEP_RECURRENCE ||
-       (o.sweep == SR_SWEEP_AUTO && (g.mode == SR_MODE_NEAR || n_om > kWave || (mean_steps >= 1008 && spread < 2048)))))
+      (o.sweep == SR_SWEEP_RECURRENCE || (o.sweep == SR_SWEEP_AUTO && pays)))
     pl.sweep = SWEEP_REC;
   // FP64: groups of threads that may share a tile's steps: blocks of at most
   // kMaxParts waves, two staged tiles of steps for each, and of the steps up to a
@@ -1063,10 +1075,8 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
   };
   int64_t chunks;
   if (pl.sweep == SWEEP_REC) {
-    // groups of 32 omegas per tile (factored.h): the number whose tiles cost
-    // least, a step of a tile costing kFactoredStage for its stage and the
-    // matrix factors of NG groups
-    const bool far = g.mode == SR_MODE_FAR;
+    // groups of 32 omegas per tile (factored.h): the number whose tiles cost least
+    // (factored_cost)
     pl.M = (far && o.omega_per_lane != 2 && o.omega_per_lane != 1) ? 4 : 2;
     const int max_groups = pl.M == 4 ? 16 : far ? 8 : 4;
     double best = INFINITY;
@@ -1088,9 +1098,13 @@ Plan make_plan(const sr_grid &g, const sr_opts &o, int64_t n_particles, uint32_t
     // wave has four stages' steps of each track: each fills queues of its own (30 x 200
     // steps on 600 x 40 x 20, three words: 0.71 ms with one, 1.08 with two; 100 x 400 on
     // 512 x 16 x 16 0.68 against 0.82); one stage each where even the tiles of two waves
-    // leave half of the CUs without one
-    auto shared = [&](int w, int stages) { return mean_steps >= (int64_t)w * stages * (kWave - 1); };
-    pl.waves = pl.groups == 16 && shared(2, 4) ? 2 : 1;
+    // leave half of the CUs without one.  Of a record's steps a wave has half a stage's
+    // or more, a second wave for 16 groups' sake four stages' (24 x 1600 steps on 512 x 12
+    // x 12, a record every 133: two waves 1.15 times one)
+    auto shared = [&](int w, int stages) {
+      return mean_steps >= (int64_t)w * stages * (kWave - 1) && record_steps >= w * (kWave / 2);
+    };
+    pl.waves = pl.groups == 16 && record_steps >= 2 * 4 * (kWave - 1) ? 2 : 1;
     while (pl.waves < 4 && ((shared(2 * pl.waves, 4) && chunks * pl.waves * spread < 2048) ||
                             (shared(2 * pl.waves, 1) && chunks * pl.waves * spread < 512)))
       pl.waves *= 2;

@@ -186,6 +186,46 @@ def test_large_far_launch_plan():
     assert rc == 0 and n == 6 * 8 * t.n_points + 4 * n_grid * 8 + 8 * 16384
 
 
+@pytest.mark.parametrize("mode,comp,n_omega,n_dir,particles,steps,snaps,factored", [
+    # one record: by the track length and how full a tile is
+    ("far", "total", 128, 144, 1000, 63, 1, False), ("far", "total", 128, 144, 1000, 64, 1, True),
+    ("far", "total", 512, 144, 1000, 31, 1, False), ("far", "total", 512, 144, 1000, 32, 1, True),
+    ("far", "total", 600, 144, 1000, 32, 1, False), ("far", "cartesian", 300, 144, 1000, 63, 1, False),
+    ("far", "cartesian_complex", 256, 144, 1000, 95, 1, False), ("far", "cartesian_complex", 256, 144, 1000, 96, 1, True),
+    ("near", "total", 128, 256, 600, 63, 1, False), ("near", "total", 128, 256, 600, 64, 1, True),
+    # several: by the steps up to a record
+    ("far", "total", 512, 144, 24, 1600, 20, True), ("far", "total", 512, 144, 24, 1600, 21, False),
+    ("far", "spheric_complex", 256, 144, 24, 1600, 16, True), ("far", "spheric_complex", 256, 144, 24, 1600, 17, False),
+    ("near", "cartesian", 128, 256, 8, 1600, 400, False),
+    # at most 64 omegas: a sine each, but for long tracks on few directions (near: or 256 steps)
+    ("far", "total", 64, 1024, 32, 4000, 1, False), ("far", "total", 24, 80, 1, 6000, 1, True),
+    ("far", "total", 24, 80, 1, 6000, 100, False), ("near", "total", 64, 256, 40, 255, 1, False),
+    ("near", "total", 64, 256, 40, 256, 1, True), ("near", "total", 64, 16, 1, 64, 1, True),
+])
+def test_plan_takes_the_faster_sweep(mode, comp, n_omega, n_dir, particles, steps, snaps, factored):
+    """SR_SWEEP_AUTO on linear grids at the lines of its rule; asked for by name, the
+    factored sweep runs either way."""
+    L = _abi.load()
+    t = _tracks(particles, n_snaps=snaps, snaps_stride=snaps)
+    t.n_points = particles * steps
+    g = _grid(mode=_abi.MODES[mode], n_omega=n_omega, n_theta=n_dir, n_phi=1, radius=FAKE, omega_step=1.0)
+    info = _abi.SrPlanInfo()
+    for sweep, want in ((_abi.SR_SWEEP_AUTO, factored), (_abi.SR_SWEEP_RECURRENCE, True), (_abi.SR_SWEEP_DIRECT, False)):
+        o = _opts(comp=_abi.COMPS[comp], sweep=sweep, form_factor=FAKE)
+        assert L.sr_plan(ctypes.byref(t), ctypes.byref(g), ctypes.byref(o), ctypes.byref(info)) == 0, _err()
+        assert (info.sweep == _abi.SR_SWEEP_RECURRENCE) == want
+
+
+@pytest.mark.parametrize("steps,snaps,waves", [(8000, 1, 2), (1600, 1, 2), (1600, 2, 2), (1600, 4, 1), (1600, 20, 1)])
+def test_plan_shares_a_record_s_steps_among_waves(steps, snaps, waves):
+    L = _abi.load()
+    t = _tracks(24, n_snaps=snaps, snaps_stride=snaps)
+    t.n_points = 24 * steps
+    info = _abi.SrPlanInfo()
+    assert L.sr_plan(ctypes.byref(t), ctypes.byref(_grid(omega_step=1.0)), ctypes.byref(_opts()), ctypes.byref(info)) == 0
+    assert info.sweep == _abi.SR_SWEEP_RECURRENCE and info.waves_per_block == waves
+
+
 def test_per_particle_entry_points_validate():
     L = _abi.load()
     P = FAKE

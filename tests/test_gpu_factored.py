@@ -12,6 +12,8 @@ product of 2^-22), at most 11 * 2^-22 = 2.6e-6 of |A_s| in all, and the FP32
 accumulation of up to 256 steps (24 additions of 2^-24 of the partial sum) adds
 1.4e-6 of the sum of |A_s|: 4e-6 of it together.
 """
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import torch
@@ -44,6 +46,7 @@ def _run(mode, comp, tracks, axes, dt, tuning=None, L_screen=None, **kw):
     ax1 = axes["theta"] if mode == "far" else axes["radius"]
     grid = engine.DeviceGrid(mode, axes["omega"], ax1, axes["phi"], L_screen=L_screen)
     assert grid.omega_step != 0.0
+    tuning = replace(tuning or engine.Tuning(), sweep="recurrence")   # short tracks too
     outs = engine.spectrum(batch, grid, comp=comp, precision="float", tuning=tuning)
     torch.cuda.synchronize()
     return {k: o.cpu().numpy().swapaxes(-1, -3) for k, o in zip(engine.COMP_KEYS[comp], outs)}
@@ -188,8 +191,8 @@ def test_small_component_keeps_its_accuracy():
 @pytest.mark.parametrize("n_steps", [1007, 1008, 1009])
 @pytest.mark.parametrize("kind,n_omega", [("up", 2), ("up", 24), ("down", 33), ("cross", 64)])
 def test_small_grids_of_long_tracks(kind, n_omega, n_steps):
-    """Grids of at most one wave's frequencies, at the track length where they take the
-    factored tiles; four waves share the steps."""
+    """Grids of at most one wave's frequencies, at the track length from which they take
+    the factored tiles by themselves; four waves share the steps."""
     test_far_edges(kind, n_omega, n_steps, 0, 0)
 
 
