@@ -1,15 +1,17 @@
 """Autotuner for the tile kernel's launch shape.
 
-For a (mode, comp, precision, grid shape) it times the candidate plans --
-sweep (direct / recurrence), omegas per thread M and waves per block (which is
-also the number of steps per LDS tile, 64 per wave) -- through the library's
-own ``sr_autotune`` (HIP events around the batch call, one untimed run per
-candidate), on a sample of the request chosen so that each tile does the work
-it does in the full launch:
+For a (mode, comp, precision, grid shape, snapshots, track length) it times the
+candidate plans -- sweep (direct / recurrence), omegas per thread M and waves per
+block -- and the library's own plan through the library's ``sr_autotune`` (HIP
+events around the batch call, one untimed run per candidate), on a sample of the
+request chosen so that each tile does the work it does in the full launch:
 
-* small launches: up to 16 of the batch's particles, cut to a common step
-  budget (about ``target_evals`` point-step evaluations per run), on the real
+* small launches: up to 32 of the batch's particles (more add no particle
+  slices), cut to a common step budget (about ``target_evals`` point-step
+  evaluations per run) with as many snapshot records per step, on the real
   grid (so the filter activity, which sets each tile's work, is the real one);
+  fewer particles where the budget would leave a track less than
+  SAMPLE_STEPS, the length up to which the plans' waves depend on it;
   when the fastest candidate runs under SHORT_LAUNCH_MS, every candidate is
   timed again over about SHORT_TIMING_MS of launches (one 0.5 ms launch per
   candidate ranked the undulator's plans within noise of each other);
@@ -53,36 +55,45 @@ DIRECTION_SHARE = 8
 SHORT_LAUNCH_MS = 5.0
 SHORT_TIMING_MS = 20.0
 MAX_REPS = 50
+# tracks are cut to fewer steps than this only when one alone exceeds the budget
+# (four waves with four stages of 63 steps each share a track from 1008 on)
+SAMPLE_STEPS = 1024
 
 
 def candidates(mode: str, precision: str, uniform: bool, n_omega: int) -> List[engine.Tuning]:
-    """Plans worth timing: FP64 sweeps directly with 1 or 2 omegas per thread;
-    split precision uses matrix products on linear grids ("recurrence": measured
-    faster there than every direct plan; M = 4 allows tiles of up to 512 omegas,
-    2 up to 256, and the waves share a tile's steps) and the direct sweep
-    otherwise.  Blocks whose omega run would leave more than a quarter of their
-    lanes idle are left out."""
+    """Plans worth timing beside the library's own.  Direct sweeps (FP64 with 1 or 2
+    omegas per thread, split grids without a constant step with up to 4): blocks
+    whose omega run would leave more than a quarter of their lanes idle are left
+    out.  Split precision on linear grids uses matrix products ("recurrence"): the
+    waves share a tile's steps, so their number leaves no omega idle; M = 4 allows
+    tiles of 512 omegas instead of 256, where there are more than 256, in blocks of
+    one or two waves (with four 24 betatron electrons on 512 x 32 x 32 take 8.45 ms
+    against 7.65, and one on 16 x 16 151 us against 155 with M = 2 and
+    four waves).  On at most 64 omegas the direct sweep is a choice there too."""
     T = engine.Tuning
+
+    def direct(ms):
+        pairs = [(m, w) for m in ms for w in (1, 2, 4)]
+        return [T(sweep="direct", omega_per_lane=m, waves_per_block=w) for m, w in pairs
+                if 64 * w * m == 64 or n_omega / (-(-n_omega // (64 * w * m)) * 64 * w * m) >= 0.75]
+
     if engine.PRECISIONS[precision] == _abi.SR_PREC_F64:
-        pairs = [("direct", m, w) for m in (1, 2) for w in (1, 2, 4)]
-    elif uniform:
-        pairs = [("recurrence", m, w) for m in ((2, 4) if mode == "far" else (2,)) for w in (1, 2, 4)]
-    else:
-        pairs = [("direct", m, w) for m in ((1, 2, 4) if mode == "far" else (1, 2)) for w in (1, 2, 4)]
-    out = []
-    for sweep, m, w in pairs:
-        run = 64 * w * m
-        chunks = -(-n_omega // run)
-        if n_omega / (chunks * run) >= 0.75 or run == 64:
-            out.append(T(sweep=sweep, omega_per_lane=m, waves_per_block=w))
-    return out
+        return direct((1, 2))
+    if not uniform:
+        return direct((1, 2, 4) if mode == "far" else (1, 2))
+    shapes = [(2, 1), (2, 2), (2, 4)] + ([(4, 1), (4, 2)] if mode == "far" and n_omega > 256 else [])
+    out = [T(sweep="recurrence", omega_per_lane=m, waves_per_block=w) for m, w in shapes]
+    return out + (direct((1, 2)) if n_omega <= 64 else [])
 
 
 def _key(batch: engine.DeviceBatch, grid: engine.DeviceGrid, comp: str, precision: str) -> str:
+    """What the fastest plan depends on: particles as far as they add slices, and the
+    steps a track sweeps to the next power of two."""
     hb = batch.host
-    size = "large" if is_large(batch, grid) else int(min(hb.n_particles, 16))
+    size = "large" if is_large(batch, grid) else int(min(hb.n_particles, 32))
+    steps = (hb.n_intervals() // max(hb.n_particles, 1)).bit_length()
     return json.dumps([grid.mode, comp, engine.PRECISIONS[precision], grid.n_omega, grid.n1, grid.n_phi,
-                       bool(grid.omega_step), int(hb.n_snaps), size])
+                       bool(grid.omega_step), int(hb.n_snaps), size, steps])
 
 
 def is_large(batch: engine.DeviceBatch, grid: engine.DeviceGrid) -> bool:
@@ -90,12 +101,17 @@ def is_large(batch: engine.DeviceBatch, grid: engine.DeviceGrid) -> bool:
 
 
 def sample_batch(hb: engine.HostBatch, n_grid: int, target_evals: float,
-                 max_particles: int = 16) -> engine.HostBatch:
-    """The first <= max_particles particles, each cut to the same step budget."""
+                 max_particles: int = 32) -> engine.HostBatch:
+    """The first <= max_particles particles, each cut to the same step budget, with the
+    batch's snapshot records per step."""
     Np = min(hb.n_particles, max_particles)
+    total = target_evals / max(n_grid, 1)
+    if Np and total / Np < SAMPLE_STEPS:
+        Np = max(1, min(Np, int(total / min(SAMPLE_STEPS, max(1, np.diff(hb.offsets).max())))))
     lengths = np.diff(hb.offsets)[:Np]
-    budget = max(8, int(target_evals / max(n_grid, 1) / max(Np, 1)))
+    budget = max(8, int(total / max(Np, 1)))
     keep = np.minimum(lengths, budget)
+    snaps = max(1, round(int(hb.n_snaps) * int(keep.sum()) / max(1, int(lengths.sum()))))
     off = np.zeros(Np + 1, dtype=np.int64)
     np.cumsum(keep, out=off[1:])
     idx = np.concatenate([np.arange(hb.offsets[p], hb.offsets[p] + keep[p]) for p in range(Np)]) \
@@ -104,9 +120,9 @@ def sample_batch(hb: engine.HostBatch, n_grid: int, target_evals: float,
     its = hb.it_start[:Np]
     if hb.snaps_stride:
         # per-track mode: each sample particle records at its own (new) end
-        return engine.pack_csr(off, *cols, hb.weight[:Np], dt=hb.dt, nSnaps=1)
+        return engine.pack_csr(off, *cols, hb.weight[:Np], dt=hb.dt, nSnaps=snaps)
     return engine.pack_csr(off, *cols, hb.weight[:Np], its, dt=hb.dt,
-                           it_range=(0, int(keep.max()) if Np else 1), nSnaps=1)
+                           it_range=(0, int(keep.max()) if Np else 1), nSnaps=snaps)
 
 
 def direction_subset(grid: engine.DeviceGrid, share: int = DIRECTION_SHARE) -> engine.DeviceGrid:
@@ -230,18 +246,24 @@ def tune(batch: engine.DeviceBatch, grid: engine.DeviceGrid, comp: str = "total"
             plan = lib_plan
     else:
         sb = engine.DeviceBatch(sample_batch(batch.host, grid.n_grid, target_evals), grid.device)
-        ms, best = time_candidates(sb, grid, comp, precision, cands)
-        record("sample", sb, grid, cands, ms)
+        timed = cands + [engine.Tuning()]   # the library's own plan last
+
+        def record_all(stage, ms):
+            record(stage, sb, grid, cands, ms)
+            record(f"{stage}, library's plan", sb, grid, timed[-1:], ms[-1:])
+
+        ms, best = time_candidates(sb, grid, comp, precision, timed)
+        record_all("sample", ms)
         # short launches (the 0.5 ms undulator spectrum): one launch per
         # candidate is within noise of the next, so time each ~20 ms again
         fastest = min((t for t in ms if np.isfinite(t) and t > 0), default=0.0)
-        if len(cands) > 1 and 0.0 < fastest < SHORT_LAUNCH_MS:
+        if 0.0 < fastest < SHORT_LAUNCH_MS:
             reps = int(min(MAX_REPS, np.ceil(SHORT_TIMING_MS / fastest)))
-            ms, best = time_candidates(sb, grid, comp, precision, cands, reps=reps, warmup=1)
-            record(f"sample x{reps}", sb, grid, cands, ms)
+            ms, best = time_candidates(sb, grid, comp, precision, timed, reps=reps, warmup=1)
+            record_all(f"sample x{reps}", ms)
         # the launch gets the winning shape; its particle slices are the
         # library's choice for the launch
-        plan = replace(cands[best], slices=0)
+        plan = replace(timed[best], slices=0)
     _cache[key] = {"plan": asdict(plan), "timings": rows}
     if path:
         try:

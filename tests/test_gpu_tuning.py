@@ -81,3 +81,21 @@ def test_large_launch_is_tuned_on_a_direction_subset():
     lib = engine.spectrum(batch, grid, comp="total", precision="float")[0]
     rel = float(torch.linalg.norm(tuned - lib) / torch.linalg.norm(lib))
     assert rel < 1e-6
+
+
+@pytest.mark.parametrize("n_omega,n_steps,nSnaps", [(24, 1500, 1), (64, 300, 1), (130, 900, 1), (180, 40, 1),
+                                                    (128, 1600, 200)])
+def test_auto_runs_and_times_the_library_s_plan(n_omega, n_steps, nSnaps):
+    """Grids of any number of omegas, short tracks and many records: the library's own plan
+    is among the timed ones, and what is chosen was not slower."""
+    wl = workloads.config2(n_particles=4, n_steps=n_steps, grid=(n_omega, 6, 5))
+    ax = wl.axes
+    grid = engine.DeviceGrid("far", ax["omega"], ax["theta"], ax["phi"])
+    batch = engine.DeviceBatch(engine.pack_tracks(wl.track_list(), dt=wl.batch.dt, nSnaps=nSnaps))
+    out = engine.spectrum(batch, grid, comp="total", precision="float", tuning="auto")[0]
+    plan, rows = autotune.tune(batch, grid, comp="total", precision="float")
+    last = [r for r in rows if r["stage"].split(",")[0] == rows[-1]["stage"].split(",")[0]]
+    assert rows[-1]["stage"].endswith("library's plan") and rows[-1]["plan"]["sweep"] == "auto"
+    assert next(r["ms"] for r in last if r["plan"] == plan.__dict__) == min(r["ms"] for r in last)
+    ref = engine.spectrum(batch, grid, comp="total", precision="double")[0]
+    assert float(torch.linalg.norm(out - ref) / torch.linalg.norm(ref)) < 1e-5

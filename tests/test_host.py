@@ -262,6 +262,51 @@ def test_autotune_candidates_and_direction_subset_rule():
     assert not large("near", 128 * 64 * 64, 500 * 3999)     # near field: tiles are not reordered
 
 
+@pytest.mark.parametrize("mode", ["far", "near"])
+@pytest.mark.parametrize("n_omega", [1, 24, 64, 65, 128, 130, 150, 180, 300, 1000])
+def test_autotune_candidates_of_linear_grids(mode, n_omega):
+    """The waves of the factored tiles share steps, so every number is a candidate
+    whatever the omegas; grids of at most 64 have the direct sweep beside it."""
+    from synchrad_amd import autotune
+    got = {(c.sweep, c.omega_per_lane, c.waves_per_block) for c in autotune.candidates(mode, "float", True, n_omega)}
+    assert {("recurrence", 2, w) for w in (1, 2, 4)} <= got
+    assert (("recurrence", 4, 2) in got) == (mode == "far" and n_omega > 256)
+    assert any(c[0] == "direct" for c in got) == (n_omega <= 64)
+    for precision, uniform in (("double", True), ("float", False)):
+        assert autotune.candidates(mode, precision, uniform, n_omega)
+
+
+def _autotune_batch(n_particles, n_steps, nSnaps=1, it_range=None):
+    off = np.arange(n_particles + 1, dtype=np.int64) * n_steps
+    cols = [np.zeros(off[-1]) for _ in range(6)]
+    return engine.pack_csr(off, *cols, np.ones(n_particles), dt=1e-3, nSnaps=nSnaps, it_range=it_range)
+
+
+def test_autotune_key_tells_plans_apart():
+    """Track lengths and particle counts that plan differently do not share a plan."""
+    from types import SimpleNamespace
+    from synchrad_amd import autotune
+    grid = SimpleNamespace(mode="far", n_omega=128, n1=8, n_phi=8, omega_step=1.0, n_grid=8192)
+    key = lambda *a, **kw: autotune._key(SimpleNamespace(host=_autotune_batch(*a, **kw)), grid, "total", "float")
+    assert len({key(16, 4000), key(32, 4000), key(16, 100), key(16, 4000, 20), key(1, 4000)}) == 5
+    assert key(40, 4000) == key(300, 3000)
+    assert key(16, 4000, 1, (0, 100)) != key(16, 4000, 1, (0, 4000))
+
+
+def test_autotune_sample_keeps_what_the_plan_depends_on():
+    from synchrad_amd import autotune
+    n_grid = 512 * 64 * 64
+    s = autotune.sample_batch(_autotune_batch(40, 8000), n_grid, 3e10)
+    assert s.n_points // s.n_particles >= 1008 and s.n_points * n_grid <= 1.1 * 3e10
+    s = autotune.sample_batch(_autotune_batch(3, 8000), 10 * n_grid, 3e10)
+    assert s.n_particles == 1 and s.n_points == int(3e10 / (10 * n_grid))
+    s = autotune.sample_batch(_autotune_batch(200, 100), n_grid, 3e10)
+    assert s.n_particles == 32 and s.n_points == 3200
+    for it_range in (None, (0, 4000)):
+        s = autotune.sample_batch(_autotune_batch(2, 4000, 40, it_range), 1 << 20, 2.0 * (1 << 20) * 2000)
+        assert s.n_points == 4000 and s.n_snaps == 20
+
+
 def _polar_spec(mode, comp="total", n=(6, 9, 8), seed=5):
     rng = np.random.default_rng(seed)
     omega = np.linspace(1.0, 4.0, n[0])
