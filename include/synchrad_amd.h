@@ -233,7 +233,10 @@ int sr_spectrum_batch_noalloc(const sr_tracks *tracks, const sr_grid *grid, cons
  * fixed.  SR_PREC_F64 evaluates everything in FP64; SR_PREC_SPLIT forms
  * phases in FP64 and sin/cos and the omega sums in FP32.  opts.slices sets the
  * number of direction groups (0 = chosen); opts.waves_per_block the block size
- * of the transpose sweep (threads = steps).  The workspace holds the group
+ * of the transpose sweep (threads = steps); opts.sweep = SR_SWEEP_DIRECT keeps
+ * long tracks on linear grids from the matrix products too, and the fields to the
+ * direct sweep (for tracks of which a window leaves little: the library sees their
+ * whole length).  The workspace holds the group
  * slabs, the particles' complex fields for a chunk of particles (at most
  * ~2 GiB; larger batches are processed chunk by chunk), the step data and, for
  * SR_PREC_SPLIT on linear grids, coefficient tables (~256 MiB, one direction of
@@ -268,8 +271,8 @@ int sr_far_fields_batch(const sr_tracks *tracks, const sr_grid *grid, const sr_o
 /*
  * sr_far_adjoint_batch with the fields of sr_far_fields_batch (same tracks,
  * grid and precision) passed in instead of recomputed: the backward of a
- * forward that kept them.  The workspace holds only the group slabs and the
- * step data.  No counterpart in the reference.
+ * forward that kept them.  The workspace holds the group slabs, the step data
+ * and the coefficient tables.  No counterpart in the reference.
  */
 int sr_far_adjoint_fields_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid,
                                           const sr_opts *opts, size_t *bytes);

@@ -109,6 +109,9 @@ def sample_batch(hb: engine.HostBatch, n_grid: int, target_evals: float,
     if Np and total / Np < SAMPLE_STEPS:
         Np = max(1, min(Np, int(total / min(SAMPLE_STEPS, max(1, np.diff(hb.offsets).max())))))
     lengths = np.diff(hb.offsets)[:Np]
+    if not hb.snaps_stride:
+        # (a window's tracks: the samples it leaves to sweep)
+        lengths = np.clip(hb.it_end[:Np].astype(np.int64) - hb.it_start[:Np], np.minimum(lengths, 1), lengths)
     budget = max(8, int(total / max(Np, 1)))
     keep = np.minimum(lengths, budget)
     snaps = max(1, round(int(hb.n_snaps) * int(keep.sum()) / max(1, int(lengths.sum()))))
@@ -117,11 +120,10 @@ def sample_batch(hb: engine.HostBatch, n_grid: int, target_evals: float,
     idx = np.concatenate([np.arange(hb.offsets[p], hb.offsets[p] + keep[p]) for p in range(Np)]) \
         if Np else np.zeros(0, dtype=np.int64)
     cols = [getattr(hb, c)[idx] for c in ("x", "y", "z", "ux", "uy", "uz")]
-    its = hb.it_start[:Np]
     if hb.snaps_stride:
         # per-track mode: each sample particle records at its own (new) end
         return engine.pack_csr(off, *cols, hb.weight[:Np], dt=hb.dt, nSnaps=snaps)
-    return engine.pack_csr(off, *cols, hb.weight[:Np], its, dt=hb.dt,
+    return engine.pack_csr(off, *cols, hb.weight[:Np], dt=hb.dt,
                            it_range=(0, int(keep.max()) if Np else 1), nSnaps=snaps)
 
 

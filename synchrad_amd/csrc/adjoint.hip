@@ -507,7 +507,7 @@ APlan adjoint_plan(const sr_tracks &t, const sr_grid &g, const sr_opts &o, bool 
   // 'cartesian', three words in two half-filled sets, 64 x 4000 on 128 x 32 x 32 21.6 ->
   // 17.2, 100 x 500 on 64 x 16 x 16 1.12 -> 1.20, 8 x 1000 on 24 x 16 x 16 0.54 -> 0.57
   const bool total = o.comp == SR_COMP_TOTAL;
-  pl.factored = split && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) && g.n_omega >= (total ? 24u : 64u);
+  pl.factored = split && o.sweep != SR_SWEEP_DIRECT && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) && g.n_omega >= (total ? 24u : 64u);
   int waves = 4;
   if (pl.factored) {
     waves = kAdjMaxT / kWave;
@@ -591,11 +591,11 @@ size_t adjoint_slab_words(const sr_tracks &t, const APlan &pl) {
 // workspace: the factored sweep's tables, slabs, the fields of one chunk of particles (unless the caller
 // passes them), the step data, and (with own fields) the fields launches' tile
 // order
-size_t adjoint_ws(const sr_tracks &t, const sr_grid &g, const APlan &pl, bool own_fields, int32_t precision) {
+size_t adjoint_ws(const sr_tracks &t, const sr_grid &g, const sr_opts &o, const APlan &pl, bool own_fields) {
   const size_t n_grid = (size_t)g.n_omega * g.n_theta * g.n_phi;
   return pl.tab_bytes + (adjoint_slab_words(t, pl) + (own_fields ? 6 * (size_t)pl.chunk * n_grid : 0) +
           6 * (size_t)t.n_points) * sizeof(double) +
-         (own_fields ? fields_order_space(t, g, precision, pl.chunk) : 0);
+         (own_fields ? fields_order_space(t, g, o, pl.chunk) : 0);
 }
 
 // the adjoint; fields_in = NULL: the fields are computed chunk by chunk in the
@@ -613,7 +613,7 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
   if (!gx || !gy || !gz || !gux || !guy || !guz || !gw) return fail(SR_ERR_INVALID, "a gradient pointer is NULL");
   const bool own = (fields_in == nullptr);
   const APlan pl = adjoint_plan(*t, *g, *o, !own);
-  const size_t need = adjoint_ws(*t, *g, pl, own, o->precision);
+  const size_t need = adjoint_ws(*t, *g, *o, pl, own);
   if (!workspace || workspace_bytes < need)
     return fail(SR_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
   AParams p;
@@ -647,7 +647,7 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
   double *fields = p.slab + adjoint_slab_words(*t, pl);
   double *pre = own ? fields + 6 * (size_t)pl.chunk * (size_t)p.n_grid : fields;
   void *order_ws = own ? (void *)(pre + 6 * (size_t)t->n_points) : nullptr;
-  const size_t order_space = own ? fields_order_space(*t, *g, o->precision, pl.chunk) : 0;
+  const size_t order_space = own ? fields_order_space(*t, *g, *o, pl.chunk) : 0;
   p.F = own ? fields : fields_in;
   p.pre = pre;
   hipStream_t st = (hipStream_t)stream;
@@ -660,7 +660,7 @@ int adjoint_run(const sr_tracks *t, const sr_grid *g, const sr_opts *o, const do
     if (own) {
       const int64_t n_f = 6 * (pe - pb) * p.n_grid;
       hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)((n_f + 255) / 256)), dim3(256), 0, st, fields, n_f);
-      if ((rc = spectrum_fields(*t, *g, o->precision, pb, pe, pre, fields, st, order_ws, order_space))) return rc;
+      if ((rc = spectrum_fields(*t, *g, *o, pb, pe, pre, fields, st, order_ws, order_space))) return rc;
     }
     p.chunk_base = pb;
     p.chunk_n = pe - pb;
@@ -705,7 +705,7 @@ int sr_far_adjoint_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid,
   int rc = adjoint_check(tracks, grid, opts);
   if (rc) return rc;
   if (tracks->n_particles == 0) return SR_OK;
-  *bytes = adjoint_ws(*tracks, *grid, adjoint_plan(*tracks, *grid, *opts, false), true, opts->precision);
+  *bytes = adjoint_ws(*tracks, *grid, *opts, adjoint_plan(*tracks, *grid, *opts, false), true);
   return SR_OK;
 }
 
@@ -722,7 +722,7 @@ int sr_far_fields_workspace_bytes(const sr_tracks *tracks, const sr_grid *grid, 
   int rc = adjoint_check(tracks, grid, opts);
   if (rc) return rc;
   *bytes = 6 * (size_t)tracks->n_points * sizeof(double) +
-           fields_order_space(*tracks, *grid, opts->precision, tracks->n_particles);
+           fields_order_space(*tracks, *grid, *opts, tracks->n_particles);
   return SR_OK;
 }
 
@@ -736,7 +736,7 @@ int sr_far_fields_batch(const sr_tracks *t, const sr_grid *g, const sr_opts *o, 
   if (outs)
     for (int c = 0; c < n_out; c++)
       if (!outs[c]) return fail(SR_ERR_INVALID, "outs[%d] is NULL", c);
-  const size_t order_space = fields_order_space(*t, *g, o->precision, t->n_particles);
+  const size_t order_space = fields_order_space(*t, *g, *o, t->n_particles);
   const size_t need = 6 * (size_t)t->n_points * sizeof(double) + order_space;
   if (!workspace || workspace_bytes < need)
     return fail(SR_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
@@ -746,7 +746,7 @@ int sr_far_fields_batch(const sr_tracks *t, const sr_grid *g, const sr_opts *o, 
   const int64_t n_f = 6 * t->n_particles * n_grid;
   hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)((n_f + 255) / 256)), dim3(256), 0, st, fields, n_f);
   if ((rc = step_prep(*t, SR_MODE_FAR, pre, st))) return rc;
-  if ((rc = spectrum_fields(*t, *g, o->precision, 0, t->n_particles, pre, fields, st,
+  if ((rc = spectrum_fields(*t, *g, *o, 0, t->n_particles, pre, fields, st,
                             (void *)(pre + 6 * (size_t)t->n_points), order_space)))
     return rc;
   if (outs)
@@ -765,7 +765,7 @@ int sr_far_adjoint_fields_workspace_bytes(const sr_tracks *tracks, const sr_grid
   int rc = adjoint_check(tracks, grid, opts);
   if (rc) return rc;
   if (tracks->n_particles == 0) return SR_OK;
-  *bytes = adjoint_ws(*tracks, *grid, adjoint_plan(*tracks, *grid, *opts, true), false, opts->precision);
+  *bytes = adjoint_ws(*tracks, *grid, *opts, adjoint_plan(*tracks, *grid, *opts, true), false);
   return SR_OK;
 }
 

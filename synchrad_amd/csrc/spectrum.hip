@@ -1454,7 +1454,7 @@ int single_particle(int32_t mode, int32_t comp, double *const *outs, const doubl
   kp.single_its = itStart;
   kp.single_ite = itEnd;
   fill_grid(kp, g, o, n_out, outs);
-  Plan pl = make_plan(g, o, 1, nSnaps, nSteps, nSteps);
+  Plan pl = make_plan(g, o, 1, nSnaps, nSteps, std::min(nSteps, itEnd));
   pl.slices = 1;  // one particle: no slices, no workspace
   slice_particles(kp, 1, 1, nullptr);
   return run(kp, pl, g, o, nullptr, 0, (hipStream_t)stream);
@@ -1483,28 +1483,29 @@ int64_t chunk_points(const sr_tracks &t, int64_t p_begin, int64_t p_end) {
   if (t.offsets_host) return t.offsets_host[p_end] - t.offsets_host[p_begin];
   return t.n_particles ? t.n_points * (p_end - p_begin) / t.n_particles : 0;
 }
-sr_opts fields_opts(int32_t precision) {
+sr_opts fields_opts(const sr_opts &request) {
   sr_opts o;
   memset(&o, 0, sizeof(o));
   o.comp = kCompField;
-  o.precision = precision;
+  o.precision = request.precision;
+  if (request.sweep == SR_SWEEP_DIRECT) o.sweep = SR_SWEEP_DIRECT;
   // every particle's field has its own output, so particle slices cost no
   // reduction: split fields take the finest tiles (the adjoint workload's
   // 256 x 4000 steps on 128 x 32 x 32: 41.4 ms at 32 slices against 42.7 at
   // the library plan's 8, heaviest first); FP64 keeps the plan (90.6 ms
   // against 93.1 at 32)
-  if (precision == SR_PREC_SPLIT) o.slices = kMaxSlices;
+  if (o.precision == SR_PREC_SPLIT) o.slices = kMaxSlices;
   return o;
 }
 }  // namespace
 
-size_t fields_order_space(const sr_tracks &t, const sr_grid &g, int32_t precision, int64_t n_particles) {
-  const Plan pl = make_plan(g, fields_opts(precision), std::max<int64_t>(n_particles, 1), 1, 0, mean_steps(t));
+size_t fields_order_space(const sr_tracks &t, const sr_grid &g, const sr_opts &request, int64_t n_particles) {
+  const Plan pl = make_plan(g, fields_opts(request), std::max<int64_t>(n_particles, 1), 1, 0, mean_steps(t));
   if (pl.blocks > kOrderMaxTiles) return 0;
   return ((size_t)pl.blocks * (sizeof(float) + sizeof(int32_t)) + 255) / 256 * 256;
 }
 
-int spectrum_fields(const sr_tracks &t, const sr_grid &g, int32_t precision, int64_t p_begin, int64_t p_end,
+int spectrum_fields(const sr_tracks &t, const sr_grid &g, const sr_opts &request, int64_t p_begin, int64_t p_end,
                     const double *pre, double *F, hipStream_t st, void *order_ws, size_t order_ws_bytes) {
   KParams kp;
   memset(&kp, 0, sizeof(kp));
@@ -1519,7 +1520,7 @@ int spectrum_fields(const sr_tracks &t, const sr_grid &g, int32_t precision, int
   kp.dt = t.dt;
   kp.n_points = t.n_points;
   kp.pre = pre;
-  const sr_opts o = fields_opts(precision);
+  const sr_opts o = fields_opts(request);
   const int64_t np = p_end - p_begin;
   const int64_t n_grid = (int64_t)g.n_omega * g.n_theta * g.n_phi;
   double *outs[kMaxOut];

@@ -89,6 +89,15 @@ class HostBatch:
         act = np.minimum(n - 1, self.it_end.astype(np.int64) - 1)
         return int(np.clip(act, 0, None).sum())
 
+    def windowed_points(self) -> Optional[int]:
+        """Samples that an it_range window leaves to sweep, where that is less than
+        half of them; else None."""
+        if self.snaps_stride or self.n_particles == 0:
+            return None
+        left = np.clip(self.it_end.astype(np.int64) - self.it_start, 1, np.diff(self.offsets).clip(1))
+        used = int(left.sum())
+        return used if 2 * used < self.n_points else None
+
 
 def pack_csr(offsets, x, y, z, ux, uy, uz, weight, it_start=None, *, dt: float,
              it_range=None, nSnaps: int = 1) -> HostBatch:
@@ -405,6 +414,41 @@ class Tuning:
     tile_order: int = 0    # 0: large far-field launches run their heaviest tiles first; 1: index order
 
 
+def _window_plan(batch: DeviceBatch, grid: DeviceGrid, opts: _abi.SrOpts) -> Optional[_abi.SrPlanInfo]:
+    """The library's plan for tracks of the length a window leaves, where that is less
+    than half of theirs: by itself the library plans for the whole tracks, of which alone
+    it knows the length (100 tracks of 1100 steps, the first 40: 128 x 16 x 16 98 us
+    against 133, 512 x 16 x 16 268 against 434)."""
+    points = batch.host.windowed_points()
+    if points is None or opts.precision != _abi.SR_PREC_SPLIT or grid.omega_step == 0.0:
+        return None
+    tr, gr, info = batch.abi(), grid.abi(), _abi.SrPlanInfo()
+    tr.n_points = points
+    _abi.check(_abi.load().sr_plan(ctypes.byref(tr), ctypes.byref(gr), ctypes.byref(opts), ctypes.byref(info)))
+    return info
+
+
+def _spectrum_opts(batch: DeviceBatch, grid: DeviceGrid, comp: str, prec: int, tuning: Optional[Tuning]) -> _abi.SrOpts:
+    tun = tuning or Tuning()
+    opts = _abi.SrOpts()
+    opts.comp = _abi.COMPS[comp]
+    opts.precision = prec
+    opts.omega_per_lane = tun.omega_per_lane
+    opts.waves_per_block = tun.waves_per_block
+    opts.slices = tun.slices
+    opts.persistent = tun.persistent
+    opts.tile_order = tun.tile_order
+    opts.sweep = SWEEPS[tun.sweep]
+    if tun == Tuning():
+        opts.form_factor = 1 if (comp == "cartesian_complex" and grid.mode == "far") else None
+        info = _window_plan(batch, grid, opts)
+        if info is not None:
+            opts.sweep, opts.omega_per_lane, opts.waves_per_block = info.sweep, info.omega_per_lane, info.waves_per_block
+            opts.slices, opts.tile_order = info.slices, 0 if info.ordered else 1
+        opts.form_factor = None
+    return opts
+
+
 def spectrum(batch: DeviceBatch, grid: DeviceGrid, comp: str = "total", precision="double",
              outs: Optional[List[torch.Tensor]] = None, sigma_particle: float = 0.0,
              tuning=None, stream=None, workspace: Optional[torch.Tensor] = None) -> List[torch.Tensor]:
@@ -438,16 +482,7 @@ def spectrum(batch: DeviceBatch, grid: DeviceGrid, comp: str = "total", precisio
     for o in outs:
         if tuple(o.shape) != shape or o.dtype != torch.float64 or not o.is_contiguous():
             raise ValueError(f"outputs must be contiguous float64 of shape {shape}")
-    tun = tuning or Tuning()
-    opts = _abi.SrOpts()
-    opts.comp = _abi.COMPS[comp]
-    opts.precision = prec
-    opts.omega_per_lane = tun.omega_per_lane
-    opts.waves_per_block = tun.waves_per_block
-    opts.slices = tun.slices
-    opts.persistent = tun.persistent
-    opts.tile_order = tun.tile_order
-    opts.sweep = SWEEPS[tun.sweep]
+    opts = _spectrum_opts(batch, grid, comp, prec, tuning)
     ff = None
     if comp == "cartesian_complex" and grid.mode == "far":
         ff = grid.form_factor(sigma_particle)
@@ -483,16 +518,8 @@ def workspace_bytes(batch: DeviceBatch, grid: DeviceGrid, comp: str = "total", p
                     tuning: Optional[Tuning] = None) -> int:
     """Bytes of workspace :func:`spectrum` needs for this request."""
     L = _abi.load()
-    tun = tuning or Tuning()
-    opts = _abi.SrOpts()
-    opts.comp = _abi.COMPS[comp]
-    opts.precision = PRECISIONS[precision] if isinstance(precision, str) else int(precision)
-    opts.omega_per_lane = tun.omega_per_lane
-    opts.waves_per_block = tun.waves_per_block
-    opts.slices = tun.slices
-    opts.persistent = tun.persistent
-    opts.tile_order = tun.tile_order
-    opts.sweep = SWEEPS[tun.sweep]
+    opts = _spectrum_opts(batch, grid, comp, PRECISIONS[precision] if isinstance(precision, str) else int(precision),
+                          tuning)
     opts.form_factor = 1 if (comp == "cartesian_complex" and grid.mode == "far") else None
     tr, gr = batch.abi(), grid.abi()
     nbytes = ctypes.c_size_t(0)
@@ -549,13 +576,23 @@ class SpectrumGraph:
         return self.outs
 
 
-def _adjoint_opts(comp, precision, tuning):
+# samples a window leaves of a track from which on its fields and its adjoint take the
+# matrix products (100 tracks of 1100 steps, fields and adjoint on 300 x 8 x 8, without
+# against with: 'total' at 150 540 us against 572, at 300 760 against 664, 'cartesian' at
+# 150 574 against 827, at 300 858 against 1039, at 600 1214 against 1274)
+WINDOW_STEPS = {"fields": 192, "total": 256, "cartesian": 512}
+
+
+def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
     tun = tuning or Tuning()
     opts = _abi.SrOpts()
     opts.comp = _abi.COMPS[comp]
     opts.precision = PRECISIONS[precision] if isinstance(precision, str) else int(precision)
     opts.waves_per_block = tun.waves_per_block
     opts.slices = tun.slices
+    points = batch.host.windowed_points()
+    if points is not None and points < WINDOW_STEPS["fields" if fields else comp] * batch.host.n_particles:
+        opts.sweep = _abi.SR_SWEEP_DIRECT
     return opts
 
 
@@ -586,7 +623,7 @@ def far_fields(batch: DeviceBatch, grid: DeviceGrid, comp: str = "total", precis
                                    for o in outs):
         raise ValueError(f"{comp} needs {n_out} contiguous float64 outputs of shape {shape}")
     fields = torch.empty((6, batch.host.n_particles, grid.n_grid), dtype=torch.float64, device=dev)
-    opts = _adjoint_opts(comp, precision, None)
+    opts = _adjoint_opts(batch, grid, comp, precision, None, fields=True)
     tr, gr = batch.abi(), grid.abi()
     nbytes = ctypes.c_size_t(0)
     _abi.check(L.sr_far_fields_workspace_bytes(ctypes.byref(tr), ctypes.byref(gr), ctypes.byref(opts),
@@ -631,7 +668,7 @@ def far_adjoint(batch: DeviceBatch, grid: DeviceGrid, dS: List[torch.Tensor], co
     if grads is None:
         grads = [torch.zeros(npts, dtype=torch.float64, device=dev) for _ in range(6)] + \
                 [torch.zeros(npart, dtype=torch.float64, device=dev)]
-    opts = _adjoint_opts(comp, precision, tuning)
+    opts = _adjoint_opts(batch, grid, comp, precision, tuning)
     tr, gr = batch.abi(), grid.abi()
     nbytes = ctypes.c_size_t(0)
     size_fn = L.sr_far_adjoint_workspace_bytes if fields is None else L.sr_far_adjoint_fields_workspace_bytes

@@ -75,9 +75,11 @@ def test_cut_steps_and_signs(lo, hi):
         _check(wl, axes, comp)
 
 
-def test_window():
+@pytest.mark.parametrize("it_range", [(0, 200), (0, 300)])
+def test_window(it_range):
+    """A window of less than half of the tracks, which takes the rotation loop, and of more."""
     wl = workloads.config2(n_particles=2, n_steps=500, grid=(40, 3, 3))
-    _check(wl, wl.axes, it_range=(0, 200))
+    _check(wl, wl.axes, it_range=it_range)
 
 
 def test_coefficients_that_are_not_finite_stay_with_the_steps_that_keep_them():

@@ -307,6 +307,37 @@ def test_autotune_sample_keeps_what_the_plan_depends_on():
         assert s.n_points == 4000 and s.n_snaps == 20
 
 
+def test_short_windows_are_planned_by_their_steps():
+    """A window that leaves little of its tracks is swept as tracks of that length are."""
+    from synchrad_amd import _abi
+    grid = engine.DeviceGrid("far", np.linspace(1.0, 2.0, 128), np.linspace(0, 0.1, 4), np.linspace(0, 6, 4), device="cpu")
+    AUTO, DIRECT, RECURRENCE = _abi.SR_SWEEP_AUTO, _abi.SR_SWEEP_DIRECT, _abi.SR_SWEEP_RECURRENCE
+
+    def plan(it_range, its=0, comp="total", precision=_abi.SR_PREC_SPLIT, tuning=None, nSnaps=1, n_steps=1100):
+        hb = _autotune_batch(5, n_steps, nSnaps, it_range)
+        hb.it_start[:] = its
+        o = engine._spectrum_opts(engine.DeviceBatch(hb, device="cpu"), grid, comp, precision, tuning)
+        return o.sweep, o.omega_per_lane, o.waves_per_block, o.slices, o.tile_order
+
+    library = (AUTO, 0, 0, 0, 0)
+    assert plan((0, 40))[0] == DIRECT and plan((0, 70))[0] == RECURRENCE
+    assert plan((0, 1100)) == library and plan(None) == library and plan((0, 1040), its=300) == library
+    assert plan((0, 90), comp="cartesian_complex")[0] == DIRECT and plan((0, 540), nSnaps=30)[0] == DIRECT
+    assert plan((0, 940), its=900) == plan((0, 40))
+    assert plan((0, 540)) == plan((0, 540), n_steps=8000)   # by the window alone
+    assert plan((0, 40), precision=_abi.SR_PREC_F64) == library
+    assert plan((0, 40), tuning=engine.Tuning(waves_per_block=2)) == (AUTO, 0, 2, 0, 0)
+
+    def adjoint(it_range, comp, fields=False):
+        batch = engine.DeviceBatch(_autotune_batch(5, 1100, 1, it_range), device="cpu")
+        return engine._adjoint_opts(batch, grid, comp, "float", None, fields).sweep
+
+    assert adjoint((0, 250), "total") == DIRECT and adjoint((0, 260), "total") == AUTO
+    assert adjoint((0, 500), "cartesian") == DIRECT and adjoint((0, 520), "cartesian") == AUTO
+    assert adjoint(None, "cartesian") == AUTO
+    assert adjoint((0, 190), "total", fields=True) == DIRECT and adjoint((0, 200), "total", fields=True) == AUTO
+
+
 def _polar_spec(mode, comp="total", n=(6, 9, 8), seed=5):
     rng = np.random.default_rng(seed)
     omega = np.linspace(1.0, 4.0, n[0])
