@@ -501,13 +501,19 @@ APlan adjoint_plan(const sr_tracks &t, const sr_grid &g, const sr_opts &o, bool 
   // threads = steps of the transpose sweep; factored: four waves, as far as the
   // tracks fill them
   const int64_t steps = t.n_particles > 0 ? t.n_points / t.n_particles : 0;
-  // matrix products from the track length on at which a direction's table is paid for:
-  // betatron beams, forward and adjoint, rotation loop -> matrix products, 'total' 100 x
-  // 500 steps on 64 x 16 x 16 1.06 -> 0.97 ms, 300 x 150 on 40 x 10 x 10 0.68 -> 0.72;
-  // 'cartesian', three words in two half-filled sets, 64 x 4000 on 128 x 32 x 32 21.6 ->
-  // 17.2, 100 x 500 on 64 x 16 x 16 1.12 -> 1.20, 8 x 1000 on 24 x 16 x 16 0.54 -> 0.57
+  // matrix products where a direction's table and the basis are paid for: by the track's
+  // length and, 'total', by its (step, omega) pairs, since the rotation loop's time follows
+  // the omegas that a step keeps and the products' hardly does.  Rotation loop over matrix
+  // products, the adjoint of kept fields on 8 x 8 directions, 30, 300 and 1000 betatron
+  // electrons (44 % of the pairs kept) and the same of an undulator (all): 'total' 24 omegas
+  // x 400 steps 0.80, 0.70, 0.56, undulator 0.86, 0.93, 0.76; 24 x 1100 1.01, 0.99, 0.67,
+  // undulator 1.15, 1.49, 1.10; 64 x 400 0.86, 0.92, 0.79, undulator 0.92, 1.33, 1.28; 128 x
+  // 400 0.93, 1.07, 0.91, undulator 1.01, 1.56, 1.46.  'cartesian', three words in two
+  // half-filled sets: 64 x 1100 0.99, 0.98, 0.78, undulator 1.22, 1.82, 1.68; 128 x 1100
+  // 1.13, 1.13, 1.01, undulator 1.42, 2.20, 2.08
   const bool total = o.comp == SR_COMP_TOTAL;
-  pl.factored = split && o.sweep != SR_SWEEP_DIRECT && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) && g.n_omega >= (total ? 24u : 64u);
+  pl.factored = split && o.sweep != SR_SWEEP_DIRECT && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) &&
+                g.n_omega >= (total ? 24u : 64u) && steps * (int64_t)g.n_omega >= 1 << 15;
   int waves = 4;
   if (pl.factored) {
     waves = kAdjMaxT / kWave;

@@ -226,6 +226,26 @@ def test_plan_shares_a_record_s_steps_among_waves(steps, snaps, waves):
     assert info.sweep == _abi.SR_SWEEP_RECURRENCE and info.waves_per_block == waves
 
 
+@pytest.mark.parametrize("comp,n_omega,steps,products", [
+    ("total", 24, 1365, False), ("total", 24, 1366, True), ("total", 64, 511, False), ("total", 64, 512, True),
+    ("total", 128, 383, False), ("total", 128, 384, True), ("total", 23, 8000, False),
+    ("cartesian", 64, 1023, False), ("cartesian", 64, 1024, True), ("cartesian", 63, 8000, False),
+])
+def test_adjoint_takes_the_faster_sweep(comp, n_omega, steps, products):
+    """The coefficient tables of the matrix products are in the workspace, and only then."""
+    L = _abi.load()
+    t = _tracks(10, snaps_stride=1)
+    t.n_points = 10 * steps
+    g = _grid(n_omega=n_omega, n_theta=8, n_phi=8, omega_step=1.0)
+    n = [ctypes.c_size_t(0), ctypes.c_size_t(0)]
+    for i, sweep in enumerate((_abi.SR_SWEEP_AUTO, _abi.SR_SWEEP_DIRECT)):
+        # (one direction group, so that both plans' slabs are alike)
+        o = _opts(comp=_abi.COMPS[comp], sweep=sweep, slices=1)
+        assert L.sr_far_adjoint_fields_workspace_bytes(ctypes.byref(t), ctypes.byref(g), ctypes.byref(o),
+                                                       ctypes.byref(n[i])) == 0, _err()
+    assert (n[0].value > n[1].value) == products and (n[0].value == n[1].value) != products
+
+
 def test_per_particle_entry_points_validate():
     L = _abi.load()
     P = FAKE

@@ -42,19 +42,21 @@ def _check(wl, axes, comp="total", tuning=None, seed=5, it_range=None, tracks=No
 @pytest.mark.parametrize("comp,n_omega", [("total", n) for n in (24, 31, 32, 33, 64, 65, 129, 257, 512, 513)] +
                          [("cartesian", n) for n in (64, 65, 129, 256, 257, 513)])
 def test_group_and_tile_edges(n_omega, comp):
-    wl = workloads.config2(n_particles=2, n_steps=400 if comp == "total" else 1050, grid=(n_omega, 3, 2))
+    # tracks long enough for the matrix products: 2^15 (step, omega) pairs
+    n_steps = max(400, 2 ** 15 // n_omega + 1) if comp == "total" else 1050
+    wl = workloads.config2(n_particles=2, n_steps=n_steps, grid=(n_omega, 3, 2))
     _check(wl, wl.axes, comp)
 
 
 @pytest.mark.parametrize("n_steps", [384, 385, 386, 512, 513, 514, 700])
 def test_step_edges(n_steps):
-    wl = workloads.config2(n_particles=3, n_steps=n_steps, grid=(48, 4, 3))
+    wl = workloads.config2(n_particles=3, n_steps=n_steps, grid=(90, 4, 3))
     _check(wl, wl.axes)
 
 
 def test_uneven_tracks():
     """Tracks shorter than a wave beside one of several blocks' runs."""
-    wl = workloads.config2(n_particles=5, n_steps=2200, grid=(48, 3, 3))
+    wl = workloads.config2(n_particles=5, n_steps=2200, grid=(54, 3, 3))
     tracks = [[c[:n] for c in t[:6]] + [t[6], 0] for t, n in zip(wl.track_list(), (2200, 1, 2, 70, 900))]
     _check(wl, wl.axes, tracks=tracks)
 
@@ -78,7 +80,7 @@ def test_cut_steps_and_signs(lo, hi):
 @pytest.mark.parametrize("it_range", [(0, 200), (0, 300)])
 def test_window(it_range):
     """A window of less than half of the tracks, which takes the rotation loop, and of more."""
-    wl = workloads.config2(n_particles=2, n_steps=500, grid=(40, 3, 3))
+    wl = workloads.config2(n_particles=2, n_steps=500, grid=(70, 3, 3))
     _check(wl, wl.axes, it_range=it_range)
 
 
