@@ -577,10 +577,12 @@ class SpectrumGraph:
 
 
 # samples a window leaves of a track from which on its fields and its adjoint take the
-# matrix products (100 tracks of 1100 steps, fields and adjoint on 300 x 8 x 8, without
-# against with: 'total' at 150 540 us against 572, at 300 760 against 664, 'cartesian' at
-# 150 574 against 827, at 300 858 against 1039, at 600 1214 against 1274)
-WINDOW_STEPS = {"fields": 192, "total": 256, "cartesian": 512}
+# matrix products ('total' of fewer than 200 omegas: always).  100 tracks of 1100 steps,
+# fields and adjoint, the first 40 and 150, without against with: 'total' 128 x 16 x 16 610
+# us against 541, 788 against 681; 300 x 8 x 8 482 against 527, 586 against 572; 512 x 16 x
+# 16 1668 against 2230, 2079 against 2472; 'cartesian' 128 x 16 x 16 674 against 730, 850
+# against 822; 512 x 16 x 16 1926 against 2963, 2357 against 3059, at 300 3971 against 3784
+WINDOW_STEPS = {"fields": 192, "total": 256, "cartesian": 256}
 
 
 def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
@@ -591,7 +593,8 @@ def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
     opts.waves_per_block = tun.waves_per_block
     opts.slices = tun.slices
     points = batch.host.windowed_points()
-    if points is not None and points < WINDOW_STEPS["fields" if fields else comp] * batch.host.n_particles:
+    if points is not None and points < WINDOW_STEPS["fields" if fields else comp] * batch.host.n_particles and \
+            (fields or comp != "total" or grid.n_omega >= 200):
         opts.sweep = _abi.SR_SWEEP_DIRECT
     return opts
 

@@ -227,8 +227,8 @@ def test_plan_shares_a_record_s_steps_among_waves(steps, snaps, waves):
 
 
 @pytest.mark.parametrize("comp,n_omega,steps,products", [
-    ("total", 24, 1365, False), ("total", 24, 1366, True), ("total", 64, 511, False), ("total", 64, 512, True),
-    ("total", 128, 383, False), ("total", 128, 384, True), ("total", 23, 8000, False),
+    ("total", 24, 833, False), ("total", 24, 834, True), ("total", 40, 499, False), ("total", 40, 500, True),
+    ("total", 64, 383, False), ("total", 64, 384, True), ("total", 23, 8000, False),
     ("cartesian", 64, 1023, False), ("cartesian", 64, 1024, True), ("cartesian", 63, 8000, False),
 ])
 def test_adjoint_takes_the_faster_sweep(comp, n_omega, steps, products):

@@ -42,8 +42,8 @@ def _check(wl, axes, comp="total", tuning=None, seed=5, it_range=None, tracks=No
 @pytest.mark.parametrize("comp,n_omega", [("total", n) for n in (24, 31, 32, 33, 64, 65, 129, 257, 512, 513)] +
                          [("cartesian", n) for n in (64, 65, 129, 256, 257, 513)])
 def test_group_and_tile_edges(n_omega, comp):
-    # tracks long enough for the matrix products: 2^15 (step, omega) pairs
-    n_steps = max(400, 2 ** 15 // n_omega + 1) if comp == "total" else 1050
+    # tracks long enough for the matrix products: 20000 (step, omega) pairs
+    n_steps = max(400, 20000 // n_omega + 1) if comp == "total" else 1050
     wl = workloads.config2(n_particles=2, n_steps=n_steps, grid=(n_omega, 3, 2))
     _check(wl, wl.axes, comp)
 
@@ -80,7 +80,7 @@ def test_cut_steps_and_signs(lo, hi):
 @pytest.mark.parametrize("it_range", [(0, 200), (0, 300)])
 def test_window(it_range):
     """A window of less than half of the tracks, which takes the rotation loop, and of more."""
-    wl = workloads.config2(n_particles=2, n_steps=500, grid=(70, 3, 3))
+    wl = workloads.config2(n_particles=2, n_steps=500, grid=(210, 3, 3))
     _check(wl, wl.axes, it_range=it_range)
 
 
@@ -107,6 +107,17 @@ def test_positions_that_are_not_finite_stay_out(comp, bad):
     track = [np.array(c) for c in wl.track_list()[0][:6]]
     track[0][[200, 777]] = bad
     _check(wl, axes, comp, tracks=[track + [1.0, 0]])
+
+
+@pytest.mark.parametrize("comp,n_omega,n_steps,it_range", [
+    ("total", 24, 400, None), ("total", 31, 500, None), ("total", 48, 390, None), ("total", 201, 1100, (0, 120)),
+    ("cartesian", 64, 1100, (0, 250)), ("cartesian", 129, 1100, (0, 200))])
+def test_long_tracks_of_few_pairs(comp, n_omega, n_steps, it_range):
+    """Few omegas, or a window of a long track: the rotation loop, restarted every 8
+    omegas.  Its phases carry FP32 roundings of at most 8 rotations and its sums those of
+    runs of 8, so the matrix products' bar holds there too."""
+    wl = workloads.config2(n_particles=3, n_steps=n_steps, grid=(n_omega, 4, 3))
+    _check(wl, dict(wl.axes, omega=np.linspace(0.1, 2.0, n_omega) * wl.axes["omega"][-1]), comp, it_range=it_range)
 
 
 def test_tables_of_several_launches():

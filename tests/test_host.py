@@ -328,13 +328,14 @@ def test_short_windows_are_planned_by_their_steps():
     assert plan((0, 40), precision=_abi.SR_PREC_F64) == library
     assert plan((0, 40), tuning=engine.Tuning(waves_per_block=2)) == (AUTO, 0, 2, 0, 0)
 
-    def adjoint(it_range, comp, fields=False):
+    def adjoint(it_range, comp, n_omega=200, fields=False):
+        grid = engine.DeviceGrid("far", np.linspace(1.0, 2.0, n_omega), np.zeros(1), np.zeros(1), device="cpu")
         batch = engine.DeviceBatch(_autotune_batch(5, 1100, 1, it_range), device="cpu")
         return engine._adjoint_opts(batch, grid, comp, "float", None, fields).sweep
 
     assert adjoint((0, 250), "total") == DIRECT and adjoint((0, 260), "total") == AUTO
-    assert adjoint((0, 500), "cartesian") == DIRECT and adjoint((0, 520), "cartesian") == AUTO
-    assert adjoint(None, "cartesian") == AUTO
+    assert adjoint((0, 250), "total", 199) == AUTO and adjoint((0, 250), "cartesian", 64) == DIRECT
+    assert adjoint((0, 260), "cartesian") == AUTO and adjoint(None, "cartesian") == AUTO
     assert adjoint((0, 190), "total", fields=True) == DIRECT and adjoint((0, 200), "total", fields=True) == AUTO
 
 
