@@ -61,9 +61,13 @@ enum { SR_PREC_F64 = 0, SR_PREC_SPLIT = 1 };
  * theorems and sums the steps as matrix products (two fp16 words per FP32
  * factor, FP32 accumulation, FP64 sums).  Both apply the |dphase| < pi filter as
  * the equivalent threshold |omega| < pi/|tau_s - tau_{s-1}|.
- * SR_SWEEP_AUTO selects it on linear grids (far field: of more than 64 omegas)
- * and the direct sweep otherwise.  The FP64 path always sweeps directly and
- * filters exactly as the reference does.
+ * SR_SWEEP_AUTO selects it on linear grids of more than 64 omegas whose tracks
+ * have enough steps up to a record (their mean length over n_snaps: 64 with one
+ * record, 32 where tiles of 512 omegas are well filled, 80 with several, 96 with
+ * six outputs); on at most 64 omegas for long tracks on too few directions to
+ * fill the GPU (far: from 1008 steps on) and in the near field from 256 steps on;
+ * the direct sweep otherwise.  The FP64 path always sweeps directly and filters
+ * exactly as the reference does.
  */
 enum { SR_SWEEP_AUTO = 0, SR_SWEEP_DIRECT = 1, SR_SWEEP_RECURRENCE = 2 };
 
@@ -130,7 +134,10 @@ typedef struct sr_opts {
                                falls back: split direct 1, 2, 4 far / 1, 2 near, else 1;
                                recurrence 2, 4 far (tiles of up to 256, 512 omegas)
                                / 2 near (128), else 2; f64 1, 2, else 1 */
-  int32_t waves_per_block;  /* 0 = tuned, else 1, 2 or 4 */
+  int32_t waves_per_block;  /* 0 = tuned, else 1, 2 or 4: waves that share a tile's
+                               omegas (recurrence: its steps).  FP64 launches short of
+                               waves put up to 16 / waves_per_block groups of such waves
+                               into a block, each sweeping a part of the steps */
   int32_t slices;           /* 0 = tuned, else 1..32 particle slices */
   int32_t persistent;       /* 0 = one block per tile; >0 = that many blocks loop over tiles */
   int32_t sweep;            /* SR_SWEEP_* */
@@ -170,8 +177,8 @@ int sr_spectrum_batch(const sr_tracks *tracks, const sr_grid *grid, const sr_opt
 
 /*
  * The plan sr_spectrum_batch resolves for a request: sweep, omegas per lane,
- * waves per block, particle slices, tiles, and whether the tiles are launched
- * heaviest first.  No counterpart in the reference (whose work-group size is
+ * waves per block (of one group of threads, see sr_opts), particle slices, tiles,
+ * and whether the tiles are launched heaviest first.  No counterpart in the reference (whose work-group size is
  * fixed, synchrad/calc.py:633-646).
  */
 typedef struct sr_plan_info {

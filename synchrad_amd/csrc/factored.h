@@ -8,9 +8,9 @@
 // so the sums over the steps s of A_s e^{i omega tau_s} at all of them are the
 // four real products P_uv[a][b] = sum_s (A_s u(alpha_a tau_s)) v(beta_b tau_s),
 // u, v in {cos, sin}: matrices of 16 rows (a) x 16 columns (b) contracted over
-// the steps.  A step then costs the sines of NG + 16 phases instead of a sine
-// or a rotation for each of the 32*NG frequencies, and the multiply-adds run on
-// the matrix cores.
+// the steps.  A step then costs four phasors and NG + 16 products of them instead of
+// a sine or a rotation for each of the 32*NG frequencies, and the multiply-adds run
+// on the matrix cores.
 //
 // FP32 in fp16 matrix instructions: every factor x is two fp16 words, x = hi +
 // lo with hi = fp16(x), lo = fp16(x - hi) (22 to 24 bits), and a product is
@@ -20,9 +20,11 @@
 // FP32 accumulators hold a few blocks of steps, then go into FP64 sums.
 //
 // Phases: per step the stage takes tau * domega/2 and the first group's centre
-// phase to revolutions in FP64 and removes whole turns; a lane's phase is one
-// FP64 FMA that adds 1.5 * 2^20, whose low mantissa word is then the fraction of
-// a turn in units of 2^-32 (signed), so no further reduction is needed.
+// phase to revolutions in FP64 and removes whole turns.  A block of steps forms, per
+// step and side (columns, rows), the phasors of the first phase p and of the spacing d
+// by FP64 polynomials, and from them e^{i (p + 4 k1 d)} and e^{i k0 d}, k1, k0 = 0..3, by
+// FP64 products, rounded to FP32 in LDS; column or row 4 k1 + k0 is the FP32 product of
+// two of these.
 //
 // The |dphase| < pi filter keeps, at step s, the K_s frequencies of smallest
 // |omega| (threshold form, as in the direct sweep; K_s by the same comparison
@@ -184,7 +186,7 @@ __device__ __forceinline__ void phasor(double rev, double *c, double *s) {
 }
 
 // waves per SIMD each variant is held to: the largest count at which nothing is
-// spilled (a spilled register costs more than the wave: with 0.3 KB of scratch per
+// spilled (16 groups without the pre-pass: two values; a spilled register costs more than the wave: with 0.3 KB of scratch per
 // lane the far kernels ran 1.5 to 3 times slower)
 template <int MODE, int NG>
 constexpr int factored_waves() {

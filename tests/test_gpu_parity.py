@@ -92,10 +92,9 @@ def test_far_total_betatron_subset(betatron4, precision, sweep, M):
 @pytest.mark.parametrize("order", ["descending", "through_zero", "log"])
 @pytest.mark.parametrize("sweep,M", [("direct", 2), ("direct", 4), ("recurrence", 2), ("recurrence", 4)])
 def test_omega_order(order, sweep, M):
-    """The filter compaction of the direct sweep assumes nothing of the omega
-    order; the recurrence sweep sorts steps only for runs of non-negative,
-    increasing omegas and keeps its masked form otherwise, and is refused
-    for grids without a constant step (log grids)."""
+    """The direct sweep assumes nothing of the omega order; the recurrence sweep takes
+    a tile's omegas in the order of ascending magnitude, in two parts where they
+    cross zero, and is refused for grids without a constant step (log grids)."""
     wl = workloads.config2(n_particles=2, n_steps=1500, grid=(96, 8, 8))
     ax = dict(wl.axes)
     om = ax["omega"]
