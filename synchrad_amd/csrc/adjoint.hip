@@ -29,7 +29,8 @@
 // non-negative linear grid: a step keeps exactly the omegas below its threshold
 // |omega|/2pi < 1/(2 |tau_s - tau_{s-1}|) (the forward's test), a prefix of the table
 // found by binary search; exp(i omega tau) walks the prefix by rotation with exp(i
-// domega tau), restarted from an FP64 phase every 32 omegas.  'total' keeps the
+// domega tau), restarted from an FP64 phase every 32 omegas.  Long tracks of few omegas:
+// the same walk in FP64, on a linear grid of any order and sign.  'total' keeps the
 // coefficients on e_theta, e_phi (F is perpendicular to n).  FP64 keeps the
 // reference's exact per-pair test and an FP64 sin/cos per pair.
 #include <hip/hip_runtime.h>
@@ -110,13 +111,15 @@ namespace {
 #endif
 
 // TWO: 'total', coefficients on e_theta (word 0) and e_phi (word 1); the
-// fields are transverse, so H F has no part along n.  FINE (split, linear grids): a
-// rotation from the FP64 step phase, restarted every 8 omegas instead of 32, and the sums
-// of 8 added up, where long tracks of few omegas or of short windows take the loop instead
-// of the matrix products, whose gradients it then matches: 300 betatron electrons x 400
-// steps on 40 x 10 x 10, error of x, ux against FP64 4.0e-7, 3.3e-6 (matrix products 4.6e-7,
-// 2.8e-6; plain loop 2.7e-6, 1.2e-5), 371 us against 316 of the plain loop and 400 of the
-// products
+// fields are transverse, so H F has no part along n.  FINE (split, linear grids of either
+// order and sign): where long tracks of few omegas, or what a window leaves of them, take
+// the loop instead of the matrix products, whose gradients it then matches or betters: the
+// kept omegas are a run, rotated over from one FP64 phasor in FP64, and the FP32 sums of 8
+// ('cartesian': 16) are added up in FP64.  300 betatron electrons x 400 steps on 40 x 10 x 10, error of x, ux
+// against FP64: matrix products 3.0e-7, 2.9e-6, plain loop 2.6e-6, 1.2e-5, this one 1e-7,
+// 2.1e-6.  Bound by the issue of FP64 FMAs and conversions; an unroll of 2 keeps 'total' at
+// four waves per SIMD (124 VGPRs; 4: 145, 24 x 300 x 400 steps on 10 x 10 308 -> 326 us),
+// 'cartesian' fits them at 4
 template <int PREC, bool TWO, bool FINE>
 __global__ void __launch_bounds__(kMaxT) k_adjoint(const AParams p) {
   constexpr bool kSplit = (PREC == SR_PREC_SPLIT);
@@ -237,7 +240,7 @@ __global__ void __launch_bounds__(kMaxT) k_adjoint(const AParams p) {
       }
     }
     __syncthreads();   // tables complete
-    const bool rot = kSplit && p.domega_rev > 0.0 && s_cw[0] >= 0.0;
+    const bool prefix = kSplit && p.domega_rev > 0.0 && s_cw[0] >= 0.0;
 
     // ---- transpose sweep: threads = steps, loop over directions and omegas ----
     for (int64_t t0 = 0; t0 < n_use; t0 += T) {
@@ -273,6 +276,9 @@ __global__ void __launch_bounds__(kMaxT) k_adjoint(const AParams p) {
                              c1 * (nv[2] - m[2]) - c2 * a[2]};
 
         Acc P[NCW], R[NCW];
+        double Pd[NCW], Rd[NCW];   // FINE: the sums over the omegas
+#pragma unroll
+        for (int c = 0; c < NCW; c++) { Pd[c] = 0; Rd[c] = 0; }
 #pragma unroll
         for (int c = 0; c < NCW; c++) { P[c] = 0; R[c] = 0; }
         auto acc_pair = [&](Acc sn, Acc cs, int j) {
@@ -294,40 +300,47 @@ __global__ void __launch_bounds__(kMaxT) k_adjoint(const AParams p) {
             }
           }
         };
-        if (rot) {
-          // the omegas this step keeps: those below its threshold (a prefix)
+        if (FINE || prefix) {
+          // the omegas this step keeps: those below its threshold, a prefix, or (FINE) the
+          // run jmin..jmax of a grid of either order and sign
           const double thr = 0.5 / fabs(tau - tau_prev);
-          int lo = 0, hi = n_om;
-          while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (s_cw[mid] < thr) lo = mid + 1; else hi = mid;
-          }
-          const int jmax = lo;
-          if constexpr (FINE) {
-            const double dr = p.domega_rev * tau;
-            double er64, ei64;
-            phasor(dr - rint(dr), &er64, &ei64);
-            const float er = (float)er64, ei = (float)ei64;
-            Acc Ps[NCW], Rs[NCW];
-#pragma unroll
-            for (int c = 0; c < NCW; c++) { Ps[c] = 0; Rs[c] = 0; }
-            for (int j0 = 0; j0 < jmax; j0 += 8) {
-              const double rv = s_cw[j0] * tau;
-              const float f = (float)(rv - rint(rv));
-              float sn = __builtin_amdgcn_sinf(f), cn = __builtin_amdgcn_cosf(f);
-              acc_pair((Acc)sn, (Acc)cn, j0);
-#pragma unroll SR_ADJ_ROT_UNROLL
-              for (int j = j0 + 1; j < min(j0 + 8, jmax); j++) {
-                const float cn2 = __builtin_fmaf(cn, er, -sn * ei);
-                sn = __builtin_fmaf(cn, ei, sn * er);
-                cn = cn2;
-                acc_pair((Acc)sn, (Acc)cn, j);
-              }
-#pragma unroll
-              for (int c = 0; c < NCW; c++) { Ps[c] += P[c]; Rs[c] += R[c]; P[c] = 0; R[c] = 0; }
+          auto first = [&](auto stays) {
+            int lo = 0, hi = n_om;
+            while (lo < hi) {
+              const int mid = (lo + hi) >> 1;
+              if (stays(s_cw[mid])) lo = mid + 1; else hi = mid;
             }
+            return lo;
+          };
+          int jmin = 0, jmax;
+          if (!FINE || prefix) {
+            jmax = first([&](double w) { return w < thr; });
+          } else if (p.domega_rev > 0.0) {
+            jmin = first([&](double w) { return !(w > -thr); });
+            jmax = first([&](double w) { return w < thr; });
+          } else {
+            jmin = first([&](double w) { return !(w < thr); });
+            jmax = first([&](double w) { return w > -thr; });
+          }
+          if constexpr (FINE) {
+            constexpr int kRun = TWO ? 8 : 16;
+            if (jmin < jmax) {
+              double er, ei, cn, sn;
+              const double dr = p.domega_rev * tau, rv = s_cw[jmin] * tau;
+              phasor(dr - rint(dr), &er, &ei);
+              phasor(rv - rint(rv), &cn, &sn);
+              for (int j0 = jmin; j0 < jmax; j0 += kRun) {
+#pragma unroll(TWO ? 2 : SR_ADJ_ROT_UNROLL)
+                for (int j = j0; j < min(j0 + kRun, jmax); j++) {
+                  acc_pair((Acc)sn, (Acc)cn, j);
+                  const double cn2 = fma(cn, er, -sn * ei);
+                  sn = fma(cn, ei, sn * er);
+                  cn = cn2;
+                }
 #pragma unroll
-            for (int c = 0; c < NCW; c++) { P[c] = Ps[c]; R[c] = Rs[c]; }
+                for (int c = 0; c < NCW; c++) { Pd[c] += (double)P[c]; Rd[c] += (double)R[c]; P[c] = 0; R[c] = 0; }
+              }
+            }
           } else {
             float er, ei, sn = 0.f, cn = 1.f;
             sincos_rev(p.domega_rev * tau, &ei, &er);
@@ -379,16 +392,17 @@ __global__ void __launch_bounds__(kMaxT) k_adjoint(const AParams p) {
           else
             om_sweep(std::integral_constant<int, 0>());
         }
+        auto sum = [&](const Acc *a, const double *b, int c) { return FINE ? b[c] : (double)a[c]; };
         double gA[3], gR[3];
         if constexpr (TWO) {
 #pragma unroll
           for (int c = 0; c < 3; c++) {
-            gA[c] = (double)P[0] * et[c] + (double)P[1] * ep[c];
-            gR[c] = (double)R[0] * et[c] + (double)R[1] * ep[c];
+            gA[c] = sum(P, Pd, 0) * et[c] + sum(P, Pd, 1) * ep[c];
+            gR[c] = sum(R, Rd, 0) * et[c] + sum(R, Rd, 1) * ep[c];
           }
         } else {
 #pragma unroll
-          for (int c = 0; c < 3; c++) { gA[c] = (double)P[c]; gR[c] = (double)R[c]; }
+          for (int c = 0; c < 3; c++) { gA[c] = sum(P, Pd, c); gR[c] = sum(R, Rd, c); }
         }
         const double rs = kSplit ? 2.0 * kPi : 1.0;   // revolutions -> radians
         const double AR = rs * (A[0] * gR[0] + A[1] * gR[1] + A[2] * gR[2]);
@@ -537,17 +551,17 @@ APlan adjoint_plan(const sr_tracks &t, const sr_grid &g, const sr_opts &o, bool 
   const int64_t steps = t.n_particles > 0 ? t.n_points / t.n_particles : 0;
   // matrix products where a direction's table and the basis are paid for: by the track's
   // length and, 'total', by its (step, omega) pairs, since the rotation loop's time follows
-  // the omegas that a step keeps and the products' hardly does.  Rotation loop over matrix
-  // products, the adjoint of kept fields on 8 x 8 directions, 30, 300 and 1000 betatron
-  // electrons (44 % of the pairs kept) and the same of an undulator (all): 'total' 24 omegas
-  // x 400 steps 0.80, 0.70, 0.56, undulator 0.86, 0.93, 0.76; 24 x 1100 1.01, 0.99, 0.67,
-  // undulator 1.15, 1.49, 1.10; 64 x 400 0.86, 0.92, 0.79, undulator 0.92, 1.33, 1.28; 128 x
-  // 400 0.93, 1.07, 0.91, undulator 1.01, 1.56, 1.46.  'cartesian', three words in two
-  // half-filled sets: 64 x 1100 0.99, 0.98, 0.78, undulator 1.22, 1.82, 1.68; 128 x 1100
-  // 1.13, 1.13, 1.01, undulator 1.42, 2.20, 2.08
-  // The rotation loop taken instead (FINE, so that the gradients lose nothing) is 1.12
-  // times the plain one's time on 24 omegas, 1.2 on 56: it meets the products at about 20000
-  // pairs
+  // the omegas that a step keeps and the products' hardly does.  Plain rotation loop over
+  // matrix products, the adjoint of kept fields on 8 x 8 directions, 30, 300 and 1000
+  // betatron electrons (44 % of the pairs kept) and the same of an undulator (all): 'total'
+  // 24 omegas x 400 steps 0.80, 0.70, 0.56, undulator 0.86, 0.93, 0.76; 24 x 1100 1.01,
+  // 0.99, 0.67, undulator 1.15, 1.49, 1.10; 64 x 400 0.86, 0.92, 0.79, undulator 0.92, 1.33,
+  // 1.28; 128 x 400 0.93, 1.07, 0.91, undulator 1.01, 1.56, 1.46.  'cartesian', three words
+  // in two half-filled sets: 64 x 1100 0.99, 0.98, 0.78, undulator 1.22, 1.82, 1.68; 128 x
+  // 1100 1.13, 1.13, 1.01, undulator 1.42, 2.20, 2.08.  The loop taken instead is the FINE
+  // one, 1.13 times the plain one's time on 24 omegas, 1.2 on 40: it meets the products at
+  // about 20000 pairs.  Direct sweep asked for: as the caller knows of windows ('cartesian'
+  // on 300 x 16 x 16, 40 of 1100 steps, 1584 -> 740 us)
   const bool total = o.comp == SR_COMP_TOTAL;
   const bool suits = split && g.omega_step != 0.0 && steps >= (total ? 384 : 1024) && g.n_omega >= (total ? 24u : 64u);
   pl.factored = suits && o.sweep != SR_SWEEP_DIRECT && steps * (int64_t)g.n_omega >= 20000;

@@ -576,13 +576,14 @@ class SpectrumGraph:
         return self.outs
 
 
-# samples a window leaves of a track from which on its fields and its adjoint take the
-# matrix products ('total' of fewer than 200 omegas: always).  100 tracks of 1100 steps,
-# fields and adjoint, the first 40 and 150, without against with: 'total' 128 x 16 x 16 610
-# us against 541, 788 against 681; 300 x 8 x 8 482 against 527, 586 against 572; 512 x 16 x
-# 16 1668 against 2230, 2079 against 2472; 'cartesian' 128 x 16 x 16 674 against 730, 850
-# against 822; 512 x 16 x 16 1926 against 2963, 2357 against 3059, at 300 3971 against 3784
-WINDOW_STEPS = {"fields": 192, "total": 256, "cartesian": 256}
+# samples a window leaves of a track from which on its fields, and the 'cartesian' adjoint
+# of WINDOW_OMEGAS and more, take the matrix products.  100 tracks of 1100 steps, adjoint of
+# kept fields, the first 40 and 150, without against with: 'cartesian' 220 x 16 x 16 597 us
+# against 921, 721 against 949; 300 x 16 x 16 737 against 1584, 901 against 1594; 300 x 6 x 6
+# 258 against 269, 281 against 272; 128 x 8 x 8 the first 150 290 against 182; 'total' 300 x 8
+# x 8 the first 40 318 against 203, 512 x 16 x 16 939 against 970, 1180 against 1127
+WINDOW_STEPS = {"fields": 192, "cartesian": 256}
+WINDOW_OMEGAS = 200
 
 
 def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
@@ -593,8 +594,8 @@ def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
     opts.waves_per_block = tun.waves_per_block
     opts.slices = tun.slices
     points = batch.host.windowed_points()
-    if points is not None and points < WINDOW_STEPS["fields" if fields else comp] * batch.host.n_particles and \
-            (fields or comp != "total" or grid.n_omega >= 200):
+    if points is not None and (fields or (comp == "cartesian" and grid.n_omega >= WINDOW_OMEGAS)) and \
+            points < WINDOW_STEPS["fields" if fields else "cartesian"] * batch.host.n_particles:
         opts.sweep = _abi.SR_SWEEP_DIRECT
     return opts
 

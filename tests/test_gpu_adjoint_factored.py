@@ -18,25 +18,26 @@ pytestmark = pytest.mark.gpu
 BARS = [2e-5] * 3 + [1e-4] * 3 + [2e-5]
 
 
-def _grads(hb, grid, G, comp, precision, tuning=None):
-    out = engine.far_adjoint(engine.DeviceBatch(hb), grid, G, comp=comp, precision=precision, tuning=tuning)
+def _grads(hb, grid, G, comp, precision, tuning=None, fields=None):
+    out = engine.far_adjoint(engine.DeviceBatch(hb), grid, G, comp=comp, precision=precision, tuning=tuning, fields=fields)
     torch.cuda.synchronize()
     return out
 
 
-def _check(wl, axes, comp="total", tuning=None, seed=5, it_range=None, tracks=None):
+def _check(wl, axes, comp="total", tuning=None, seed=5, it_range=None, tracks=None, exact_fields=False, bars=BARS):
     grid = engine.DeviceGrid("far", axes["omega"], axes["theta"], axes["phi"])
     hb = engine.pack_tracks(tracks or wl.track_list(), dt=wl.batch.dt, it_range=it_range)
     rng = np.random.default_rng(seed)
     shape = (1, axes["phi"].size, axes["theta"].size, axes["omega"].size)
     G = [torch.from_numpy(rng.standard_normal(shape)).cuda() for _ in range(1 if comp == "total" else 3)]
-    got = _grads(hb, grid, G, comp, "float", tuning)
+    fields = engine.far_fields(engine.DeviceBatch(hb), grid, comp=comp, precision="double")[0] if exact_fields else None
+    got = _grads(hb, grid, G, comp, "float", tuning, fields)
     ref = _grads(hb, grid, G, comp, "double")
     for c in range(7):
         n = float(torch.linalg.norm(ref[c]))
         r = float(torch.linalg.norm(got[c] - ref[c])) / n if n > 0 else 0.0
         print(f"{comp} grad[{c}]: rel-L2 {r:.3e}", flush=True)
-        assert r <= BARS[c], (c, r)
+        assert r <= bars[c], (c, r)
 
 
 @pytest.mark.parametrize("comp,n_omega", [("total", n) for n in (24, 31, 32, 33, 64, 65, 129, 257, 512, 513)] +
@@ -77,11 +78,11 @@ def test_cut_steps_and_signs(lo, hi):
         _check(wl, axes, comp)
 
 
-@pytest.mark.parametrize("it_range", [(0, 200), (0, 300)])
-def test_window(it_range):
-    """A window of less than half of the tracks, which takes the rotation loop, and of more."""
-    wl = workloads.config2(n_particles=2, n_steps=500, grid=(210, 3, 3))
-    _check(wl, wl.axes, it_range=it_range)
+@pytest.mark.parametrize("comp,n_steps,it_range", [
+    ("total", 500, (0, 200)), ("total", 500, (0, 300)), ("cartesian", 1100, (0, 260))])
+def test_window(comp, n_steps, it_range):
+    wl = workloads.config2(n_particles=2, n_steps=n_steps, grid=(210, 3, 3))
+    _check(wl, wl.axes, comp, it_range=it_range)
 
 
 def test_coefficients_that_are_not_finite_stay_with_the_steps_that_keep_them():
@@ -109,15 +110,22 @@ def test_positions_that_are_not_finite_stay_out(comp, bad):
     _check(wl, axes, comp, tracks=[track + [1.0, 0]])
 
 
+@pytest.mark.parametrize("order", ["up", "down", "cross"])
 @pytest.mark.parametrize("comp,n_omega,n_steps,it_range", [
-    ("total", 24, 400, None), ("total", 31, 500, None), ("total", 48, 390, None), ("total", 201, 1100, (0, 120)),
-    ("cartesian", 64, 1100, (0, 250)), ("cartesian", 129, 1100, (0, 200))])
-def test_long_tracks_of_few_pairs(comp, n_omega, n_steps, it_range):
-    """Few omegas, or a window of a long track: the rotation loop, restarted every 8
-    omegas.  Its phases carry FP32 roundings of at most 8 rotations and its sums those of
-    runs of 8, so the matrix products' bar holds there too."""
+    ("total", 24, 400, None), ("total", 31, 500, None), ("total", 48, 390, None),
+    ("cartesian", 201, 1100, (0, 120)), ("cartesian", 513, 1100, (0, 250))])
+def test_long_tracks_of_few_pairs(comp, n_omega, n_steps, it_range, order):
+    """Few omegas, or a window of a long track: the rotation loop in FP64, here of FP64 fields.
+    What a position's gradient sums is rounded to FP32 in the coefficient, the frequency, the
+    sine, the cosine, two products and a run's sum: 8 roundings of 2^-24 bound it; the
+    momenta's sums over the track cancel to a twentieth of their terms.  The weights' are
+    FP64."""
     wl = workloads.config2(n_particles=3, n_steps=n_steps, grid=(n_omega, 4, 3))
-    _check(wl, dict(wl.axes, omega=np.linspace(0.1, 2.0, n_omega) * wl.axes["omega"][-1]), comp, it_range=it_range)
+    top = wl.axes["omega"][-1]
+    omega = {"up": np.linspace(0.1, 2.0, n_omega), "down": np.linspace(2.0, 0.1, n_omega),
+             "cross": np.linspace(-2.0, 2.0, n_omega)}[order] * top
+    _check(wl, dict(wl.axes, omega=omega), comp, it_range=it_range, exact_fields=True,
+           bars=[5e-7] * 3 + [1e-5] * 3 + [1e-12])
 
 
 def test_tables_of_several_launches():

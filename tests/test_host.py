@@ -333,9 +333,9 @@ def test_short_windows_are_planned_by_their_steps():
         batch = engine.DeviceBatch(_autotune_batch(5, 1100, 1, it_range), device="cpu")
         return engine._adjoint_opts(batch, grid, comp, "float", None, fields).sweep
 
-    assert adjoint((0, 250), "total") == DIRECT and adjoint((0, 260), "total") == AUTO
-    assert adjoint((0, 250), "total", 199) == AUTO and adjoint((0, 250), "cartesian", 64) == DIRECT
-    assert adjoint((0, 260), "cartesian") == AUTO and adjoint(None, "cartesian") == AUTO
+    assert adjoint((0, 250), "cartesian") == DIRECT and adjoint((0, 260), "cartesian") == AUTO
+    assert adjoint((0, 250), "cartesian", 199) == AUTO and adjoint((0, 40), "total") == AUTO
+    assert adjoint(None, "cartesian") == AUTO and adjoint((0, 190), "cartesian", 64, fields=True) == DIRECT
     assert adjoint((0, 190), "total", fields=True) == DIRECT and adjoint((0, 200), "total", fields=True) == AUTO
 
 
