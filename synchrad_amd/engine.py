@@ -576,14 +576,20 @@ class SpectrumGraph:
         return self.outs
 
 
-# samples a window leaves of a track from which on its fields, and the 'cartesian' adjoint
-# of WINDOW_OMEGAS and more, take the matrix products.  100 tracks of 1100 steps, adjoint of
-# kept fields, the first 40 and 150, without against with: 'cartesian' 220 x 16 x 16 597 us
-# against 921, 721 against 949; 300 x 16 x 16 737 against 1584, 901 against 1594; 300 x 6 x 6
-# 258 against 269, 281 against 272; 128 x 8 x 8 the first 150 290 against 182; 'total' 300 x 8
-# x 8 the first 40 318 against 203, 512 x 16 x 16 939 against 970, 1180 against 1127
-WINDOW_STEPS = {"fields": 192, "cartesian": 256}
-WINDOW_OMEGAS = 200
+def _window_steps(comp: str, n_omega: int, fields: bool) -> int:
+    """Samples a window leaves of a track from which on its fields, and its adjoint, take
+    the matrix products.  100 tracks of 1100 steps, without against with.  Fields: 128 x 16 x
+    16 the first 40 178 us against 230, 150 317 against 298; 200 x 16 x 16 90 342 against 390,
+    150 470 against 440; 256 x 16 x 16 60 384 against 495, 190 609 against 578 (x 8 x 8 60 142
+    against 141, 90 159 against 151); from 257 omegas on tiles of 512, 300 x 8 x 8 190 264
+    against 382, 250 315 against 385; 512 x 16 x 16 250 1249 against 1415.  Adjoint of kept
+    fields, the first 40 and 150: 'cartesian' 220 x 16 x 16 597 against 921, 721 against 949;
+    300 x 16 x 16 737 against 1584, 901 against 1594; 300 x 6 x 6 258 against 269, 281 against
+    272; 128 x 8 x 8 150 290 against 182; 'total' 300 x 8 x 8 40 318 against 203, 512 x 16 x 16
+    939 against 970, 1180 against 1127."""
+    if fields:
+        return 96 if n_omega <= 256 else 256
+    return 256 if comp == "cartesian" and n_omega >= 200 else 0
 
 
 def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
@@ -594,8 +600,7 @@ def _adjoint_opts(batch, grid, comp, precision, tuning, fields=False):
     opts.waves_per_block = tun.waves_per_block
     opts.slices = tun.slices
     points = batch.host.windowed_points()
-    if points is not None and (fields or (comp == "cartesian" and grid.n_omega >= WINDOW_OMEGAS)) and \
-            points < WINDOW_STEPS["fields" if fields else "cartesian"] * batch.host.n_particles:
+    if points is not None and points < _window_steps(comp, grid.n_omega, fields) * batch.host.n_particles:
         opts.sweep = _abi.SR_SWEEP_DIRECT
     return opts
 

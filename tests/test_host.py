@@ -335,8 +335,9 @@ def test_short_windows_are_planned_by_their_steps():
 
     assert adjoint((0, 250), "cartesian") == DIRECT and adjoint((0, 260), "cartesian") == AUTO
     assert adjoint((0, 250), "cartesian", 199) == AUTO and adjoint((0, 40), "total") == AUTO
-    assert adjoint(None, "cartesian") == AUTO and adjoint((0, 190), "cartesian", 64, fields=True) == DIRECT
-    assert adjoint((0, 190), "total", fields=True) == DIRECT and adjoint((0, 200), "total", fields=True) == AUTO
+    assert adjoint(None, "cartesian") == AUTO and adjoint((0, 90), "cartesian", 64, fields=True) == DIRECT
+    assert adjoint((0, 90), "total", 256, fields=True) == DIRECT and adjoint((0, 100), "total", 256, fields=True) == AUTO
+    assert adjoint((0, 250), "total", 257, fields=True) == DIRECT and adjoint((0, 260), "total", 257, fields=True) == AUTO
 
 
 def _polar_spec(mode, comp="total", n=(6, 9, 8), seed=5):
